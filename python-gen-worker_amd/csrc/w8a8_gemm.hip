@@ -1,12 +1,13 @@
-// W8A8 GEMM: int8 MFMA 32x32x32 with int32 accumulation over the whole K and
+// W8A8 GEMM: int8 MFMA with int32 accumulation over the whole K and
 // the fp32 epilogue acc * sa * sw[n] + bias[n] of torch._scaled_mm: per-token
 // activation scales in the rowwise mode (models/w8a8.py:374-378), one scalar in
 // the pertensor mode (:366-372, whose weight scale and bias the reference
 // applies as two further bf16 ops; here they are fused in fp32).
 //
 // Same orientation as the W4A4 kernel: A operand = weight rows (n), B operand
-// = activation rows (m); accumulator block D[n][m], lane l holds m = l % 32
-// and n = 8*(v/4) + 4*(l/32) + (v%4).
+// = activation rows (m); a 32 x 32 accumulator block D[n][m] holds m = l % 32
+// and n = 8*(v/4) + 4*(l/32) + (v%4) in lane l, a 16 x 16 one m = l % 16 and
+// n = 4*(l/16) + v.
 #include <atomic>
 
 #include "fp6_gemm_common.h"
@@ -168,10 +169,22 @@ __global__ __launch_bounds__(256) void w8a8_gemm_kernel(const int8_t* __restrict
 // rows past M or N read zeros through the range-checked per-lane offset and the stage advance rides in the
 // scalar offset. In LDS the 16-byte chunk c of row r sits at slot c ^ ((r / 2) % 8) of the row, so the 16
 // rows a quarter of a read instruction touches fill all banks. 8 waves form a 2 (n) x 4 (m) grid of
-// 128 x 64 wave tiles: per k-step of 32 bytes, 6 operand reads feed 8 int8 MFMAs that accumulate in place.
-// The loop is software-pipelined: the reads of k-step s + 1 are issued between the MFMAs of k-step s, and
-// at a stage boundary the wave waits for its copies, meets the barrier, issues the copies two stages ahead
-// into the buffer just drained and reads the next stage's first k-step under the last k-step's MFMAs.
+// 128 x 64 wave tiles: per k-step of 64 bytes, 12 operand reads feed 32 int8 MFMAs.
+//
+// What bounds it: with operands of full range, power (4096^3 takes 44.1 us on zeros and 52.5 on normal data; the
+// clock falls as more of the chip is busy), so the form that moves the fewest register bytes wins; with the
+// small codes that outlier channels leave, the matrix pipe (85 % busy in the loop), the epilogue and the last
+// round's idle CUs. The 16 x 16 x 64 MFMA reads and writes a quarter of the sums per instruction that
+// 32 x 32 x 32 does, for half the multiply-adds: the same loop on it ran 62 -> 56 us at 4096^3, and visiting
+// the blocks in a snake, so that neighbouring MFMAs always share an operand, took another 1 %.
+//
+// The two waves of a SIMD alternate: waves 0..3 run one phase ahead of waves 4..7, and in every phase one
+// group issues a k-step's 32 MFMAs (512 matrix-pipe cycles, raised priority) while the other reads its next
+// k-step's operands into registers and issues its copies; a barrier ends each phase. Against both waves
+// running the same read-under-MFMA pipeline this took 118.6 -> 114.1 us at 4608 x 9216 x 3072. Persistent
+// workgroups that prefetch the next tile under the epilogue measured 118 us there (the epilogue's phase runs
+// beside one MFMA phase only). In all, against the 32 x 32 x 32 pipeline before it, normal data: 4096^3
+// 60.1 -> 52.5 us (2620 TOPS), 4608 x 9216 x 3072 122.1 -> 108.9, 4608 x 3072 x 3072 41.4 -> 38.
 // ---------------------------------------------------------------------------
 constexpr int L_TM = 256, L_TN = 256, L_KS = 128;  // tile rows (m, n); K bytes per stage
 constexpr int kCus = 256;                          // MI355X compute units
@@ -179,22 +192,14 @@ constexpr int L_REG = 256 * L_KS;                  // one operand region of a st
 constexpr int L_STAGE = 2 * L_REG;                 // activation region, then weight region
 constexpr int L_RUNS = L_REG / 1024;               // 1 KB copies per operand and stage: 32
 constexpr int L_SLOTS = L_STAGE / 1024 / NWAVES;   // copies per wave and stage: 8 (4 activation, 4 weight)
-constexpr int L_OSTR = L_TN * 2 + 8;              // output staging row: 8-byte pad, distinct banks per write
-constexpr int L_LDS = 2 * L_STAGE > L_TM * L_OSTR ? 2 * L_STAGE : L_TM * L_OSTR;
+constexpr int L_LDS = 2 * L_STAGE;
 static_assert(L_LDS <= kLdsBytes && L_SLOTS * NWAVES * 1024 == L_STAGE, "stage layout");
+static_assert(NWAVES * 64 * 256 <= L_LDS, "output staging");
 
 __device__ __forceinline__ int l_swz(int r) { return (r >> 1) & 7; }
 
-// pins the order of one k-step: MFMA and operand read alternate (6 reads under 8 MFMAs)
-__device__ __forceinline__ void pin_kstep() {
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-  }
-  __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-  __builtin_amdgcn_sched_barrier(0);
-}
+// s_waitcnt lgkmcnt(0), vmcnt and expcnt left at their maxima
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
 template <int BIAS_DT, bool OUT_F16>
 __global__ __launch_bounds__(NTHREADS, 1) void w8a8_gemm_lds_kernel(const int8_t* __restrict__ qa,
@@ -214,7 +219,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void w8a8_gemm_lds_kernel(const int8_t
   const int nst = K / L_KS;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wn = wave & 1, wm = wave >> 1;
-  const int r32 = lane & 31, h = lane >> 5;
+  const int r16 = lane & 15, q4 = lane >> 4;
 
   // descriptors over this tile's rows only (256 K < 2^31 bytes, checked on the host, so kOOB lies past them)
   const v4i xbuf = raw_rsrc(qa + (int64_t)m0 * K, (uint32_t)(min(M - m0, L_TM) * K));
@@ -242,44 +247,44 @@ __global__ __launch_bounds__(NTHREADS, 1) void w8a8_gemm_lds_kernel(const int8_t
       dma16(j < L_SLOTS / 2 ? xbuf : wbuf, ldst[j] + (uint32_t)(u * L_STAGE), voff[j], soff);
   };
 
-  v16i acc[4][2];
+  v4i acc[8][4], a[8], b[4];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int bn = 0; bn < 8; ++bn)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = (v16i){};
-  // operand rows of this lane: weight block bn row 128 wn + 32 bn + r32, activation block bm row 64 wm + 32 bm + r32
-  int wrow[4], xrow[2];
+    for (int bm = 0; bm < 4; ++bm) acc[bn][bm] = (v4i){};
+  // this lane's chunk of an operand row at k-step ks (64 bytes): the rows of a wave differ by multiples of 16, so
+  // the chunk swizzle is the lane's own
+  uint32_t xoff[2], woff[2];
 #pragma unroll
-  for (int bn = 0; bn < 4; ++bn) wrow[bn] = 128 * wn + 32 * bn + r32;
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t c = 16u * (uint32_t)((4 * ks + q4) ^ l_swz(r16));
+    xoff[ks] = (uint32_t)((64 * wm + r16) * L_KS) + c;
+    woff[ks] = (uint32_t)(L_REG + (128 * wn + r16) * L_KS) + c;
+  }
+  auto read_ops = [&](const uint8_t* buf, int ks) __attribute__((always_inline)) {
 #pragma unroll
-  for (int bm = 0; bm < 2; ++bm) xrow[bm] = 64 * wm + 32 * bm + r32;
-  // k-step ks (32 bytes) of a stage buffer: this lane's half h of each operand row
-  auto read_ops = [&](const uint8_t* buf, int ks, v4i (&a)[4], v4i (&b)[2]) __attribute__((always_inline)) {
-    const int c = 2 * ks + h;
+    for (int bm = 0; bm < 4; ++bm) b[bm] = *(const v4i*)(buf + xoff[ks] + bm * 16 * L_KS);
 #pragma unroll
-    for (int bn = 0; bn < 4; ++bn) a[bn] = *(const v4i*)(buf + L_REG + wrow[bn] * L_KS + 16 * (c ^ l_swz(wrow[bn])));
-#pragma unroll
-    for (int bm = 0; bm < 2; ++bm) b[bm] = *(const v4i*)(buf + xrow[bm] * L_KS + 16 * (c ^ l_swz(xrow[bm])));
+    for (int bn = 0; bn < 8; ++bn) a[bn] = *(const v4i*)(buf + woff[ks] + bn * 16 * L_KS);
   };
-  auto mma = [&](const v4i (&a)[4], const v4i (&b)[2]) __attribute__((always_inline)) {
+  // one k-step; empty asm on its operands and sums keeps the (pure) MFMAs between the phase's two barriers
+  auto mma = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]));
+    asm volatile("" : "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(b[2]), "+v"(b[3]));
+    __builtin_amdgcn_s_setprio(1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int bn = 0; bn < 4; ++bn)
+    for (int bn = 0; bn < 8; ++bn)
 #pragma unroll
-      for (int bm = 0; bm < 2; ++bm)
-        acc[bn][bm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[bn], b[bm], acc[bn][bm], 0, 0, 0);
-  };
-  // k-steps 1..3 of a stage, each read under the previous k-step's MFMAs; leaves k-step 3 in (a1, b1)
-  v4i a0[4], b0[2], a1[4], b1[2];
-  auto stage_body = [&](const uint8_t* buf) __attribute__((always_inline)) {
-    read_ops(buf, 1, a1, b1);
-    mma(a0, b0);
-    pin_kstep();
-    read_ops(buf, 2, a0, b0);
-    mma(a1, b1);
-    pin_kstep();
-    read_ops(buf, 3, a1, b1);
-    mma(a0, b0);
-    pin_kstep();
+      for (int i = 0; i < 4; ++i) {
+        const int bm = bn & 1 ? 3 - i : i;
+        acc[bn][bm] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[bn], b[bm], acc[bn][bm], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int bn = 0; bn < 8; ++bn)
+      asm volatile("" : "+v"(acc[bn][0]), "+v"(acc[bn][1]), "+v"(acc[bn][2]), "+v"(acc[bn][3]));
   };
 
   issue(0, 0);
@@ -299,75 +304,78 @@ __global__ __launch_bounds__(NTHREADS, 1) void w8a8_gemm_lds_kernel(const int8_t
   wait_vm_lgkm0<0>();
   barrier_lds();
   if (1 < nst) issue(1, 1);
-  read_ops(g_lds, 0, a0, b0);
-  for (int st = 0; st < nst - 1; ++st) {
-    stage_body(g_lds + (st & 1) * L_STAGE);
-    // stage st + 1's copies (this wave's: the only ones in flight) and this wave's reads of stage st are
-    // complete; after the barrier everyone's are, so buffer st & 1 takes the copies of stage st + 2
-    wait_vm_lgkm0<0>();
-    barrier_lds();
-    if (st + 2 < nst) issue(st & 1, st + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    read_ops(g_lds + ((st + 1) & 1) * L_STAGE, 0, a0, b0);
-    mma(a1, b1);
-    pin_kstep();
-  }
-  stage_body(g_lds + ((nst - 1) & 1) * L_STAGE);
-  mma(a1, b1);
-
-  // epilogue: y = acc * sa[m] * sw[n] + bias[n] (sw and bias from the tile's LDS copy: per-element global
-  // loads of them would cost the texture path two 64-lane instructions per output pair), packed to 16 bits and
-  // staged in LDS as [m][n] rows of OSTR
-  // bytes (the stage buffers are free once every wave has passed the barrier), then stored as whole row
-  // segments, consecutive threads on consecutive 16-byte chunks of a row (a 32-row column of 8-byte pieces
-  // per store instruction, as the accumulator layout gives, spreads every store over 32 rows of the output)
-  uint8_t* ob = g_lds;
-  barrier_lds();
+  // Every group's phases are read, MFMA, read, MFMA for each stage, waves 4..7 one phase late. The copies of
+  // stage st + 1 are issued in the first read phase of stage st, when every wave has drained that buffer (the late
+  // group's reads of stage st - 1 ended before the last barrier), and each wave waits for its own before the
+  // barrier that precedes the early group's first read of stage st + 1.
+  const bool early = wave < NWAVES / 2;
+  if (!early) barrier_lds();
+  for (int st = 0; st < nst; ++st) {
+    const uint8_t* buf = g_lds + (st & 1) * L_STAGE;
 #pragma unroll
-  for (int bm = 0; bm < 2; ++bm) {
-    const int ml = 64 * wm + 32 * bm + r32, m = m0 + ml;
-    const float am = sa[sa_row ? min(m, M - 1) : 0];  // rows past M are computed but never stored
-#pragma unroll
-    for (int bn = 0; bn < 4; ++bn) {
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int nl = 128 * wn + 32 * bn + 8 * qd + 4 * h, n = n0 + nl;
-        if (n >= N) continue;  // N % 16 == 0: n < N covers n + 3
-        const v4f cw = *(const v4f*)(g_epi + nl);
-        const v4f cb = *(const v4f*)(g_epi + L_TN + nl);
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float y = (float)acc[bn][bm][4 * qd + e] * am * cw[e];
-          if (BIAS_DT >= 0) y += cb[e];
-          o[e] = y;
-        }
-        uint2 pk;
-        if (OUT_F16) {
-          pk.x = pack_f16x2(o[0], o[1]);
-          pk.y = pack_f16x2(o[2], o[3]);
-        } else {
-          pk.x = pack_bf16x2_rn(o[0], o[1]);
-          pk.y = pack_bf16x2_rn(o[2], o[3]);
-        }
-        *(uint2*)(ob + ml * L_OSTR + nl * 2) = pk;
-      }
+    for (int ks = 0; ks < 2; ++ks) {
+      read_ops(buf, ks);
+      if (ks == 0 && st >= 1 && st + 1 < nst) issue((st + 1) & 1, st + 1);
+      if (ks == 1 && !early) wait_vm_lgkm0<0>();
+      else wait_lgkm0();
+      __builtin_amdgcn_sched_barrier(0);
+      barrier_lds();
+      mma();
+      if (ks == 1 && early) wait_vm_lgkm0<0>();
+      barrier_lds();
     }
   }
+  if (early) barrier_lds();
+
+  // epilogue: y = acc * sa[m] * sw[n] + bias[n], packed to 16 bits. Every wave stages its own 64 x 128 tile in its
+  // own 16 KB of the stage buffers (free once every wave has passed the barrier), so no barrier stands between
+  // the arithmetic and the stores, which take 256-byte row segments (four rows a store instruction; as the
+  // accumulators lie, a store would touch 16 rows' 32-byte pieces). The 16-byte chunk c of row r lies at slot
+  // c ^ (r % 16). The per-column constants are read once per column block. Against one staged tile for the
+  // workgroup, with the constants read again for every row block: 53.9 -> 52.5 us at 4096^3 (one round of tiles),
+  // 113.2 -> 108.9 at 4608 x 9216 x 3072 (three).
+  uint8_t* const stag = g_lds + wave * (64 * 256);
   barrier_lds();
-  // a descriptor over this tile's output span (255 N + 256 elements < 2^29: N < 2^21 is checked on the host)
-  const int rows = min(M - m0, L_TM), cols = min(N - n0, L_TN);
-  const rsrc_t obuf = make_rsrc(out + (int64_t)m0 * N + n0, (uint32_t)(((rows - 1) * N + cols) * 2));
-  constexpr int CPR = L_TN / 8;  // 16-byte chunks per row
-#pragma unroll 4
-  for (int i = tid; i < L_TM * CPR; i += NTHREADS) {
-    const int row = i / CPR, c = i % CPR;
-    const uint2 lo = *(const uint2*)(ob + row * L_OSTR + c * 16);
-    const uint2 hi = *(const uint2*)(ob + row * L_OSTR + c * 16 + 8);
-    uint32_t off = row < rows && 8 * c < cols ? (uint32_t)((row * N + 8 * c) * 2) : kOOB;
-    if (!GWA_DCHECK(off == kOOB || (int64_t)off + 16 <= (int64_t)((rows - 1) * N + cols) * 2, kDbgW8Out, off))
-      off = kOOB;
-    buf_store16((v4i){(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y}, obuf, off);
+  float am[4];
+#pragma unroll
+  for (int bm = 0; bm < 4; ++bm)  // rows past M are computed but never stored
+    am[bm] = sa[sa_row ? min(m0 + 64 * wm + 16 * bm + r16, M - 1) : 0];
+#pragma unroll
+  for (int bn = 0; bn < 8; ++bn) {
+    const v4f cw = *(const v4f*)(g_epi + 128 * wn + 16 * bn + 4 * q4);
+    const v4f cb = *(const v4f*)(g_epi + L_TN + 128 * wn + 16 * bn + 4 * q4);
+#pragma unroll
+    for (int bm = 0; bm < 4; ++bm) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float y = (float)acc[bn][bm][e] * am[bm] * cw[e];
+        if (BIAS_DT >= 0) y += cb[e];
+        o[e] = y;
+      }
+      uint2 pk;
+      if (OUT_F16) {
+        pk.x = pack_f16x2(o[0], o[1]);
+        pk.y = pack_f16x2(o[2], o[3]);
+      } else {
+        pk.x = pack_bf16x2_rn(o[0], o[1]);
+        pk.y = pack_bf16x2_rn(o[2], o[3]);
+      }
+      *(uint2*)(stag + (16 * bm + r16) * 256 + 16 * ((2 * bn + (q4 >> 1)) ^ r16) + 8 * (q4 & 1)) = pk;
+    }
+  }
+  asm volatile("" ::: "memory");
+  // a descriptor over the wave's output span (63 N + 128 elements < 2^28: N < 2^21 is checked on the host)
+  const int rows = min(M - m0 - 64 * wm, 64), cols = min(N - n0 - 128 * wn, 128);
+  const uint32_t span = rows > 0 && cols > 0 ? (uint32_t)(((rows - 1) * N + cols) * 2) : 0u;
+  const rsrc_t obuf = make_rsrc(out + (int64_t)(m0 + 64 * wm) * N + n0 + 128 * wn, span);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int row = 4 * i + q4;
+    const v4i v = *(const v4i*)(stag + row * 256 + 16 * (r16 ^ (row & 15)));
+    uint32_t off = row < rows && 8 * r16 < cols ? (uint32_t)((row * N + 8 * r16) * 2) : kOOB;
+    if (!GWA_DCHECK(off == kOOB || (int64_t)off + 16 <= (int64_t)span, kDbgW8Out, off)) off = kOOB;
+    buf_store16(v, obuf, off);
   }
 }
 
