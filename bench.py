@@ -424,7 +424,7 @@ def bench_w8a8(args) -> int:
         ops_ = w4a4_int_ops(m, n, k)
         row = {"M": m, "N": n, "K": k, "tile": int(lib.gwa_w8a8_gemm_tile(m, n, k))}
         qwt = qw.t()  # torch._int_mm's [K, N] operand, column-major as hipBLASLt takes it
-        variants = {"tile_128x128": 0, "tile_256x256": 1, "chosen": -1, "bf16": None, "torch_int_mm": "int_mm"}
+        variants = {"tile_128x128": 0, "tile_256x256": 1, "tile_64x64": 2, "tile_64x128": 3, "chosen": -1, "bf16": None, "torch_int_mm": "int_mm"}
         for name, tile in variants.items():
             if tile is None:
                 fn = lambda: torch.nn.functional.linear(xd, wd, bias)  # noqa: E731

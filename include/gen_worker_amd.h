@@ -435,16 +435,16 @@ int gwa_w8a8_gemm(const int8_t* qa, const int8_t* qw, const float* sa, int64_t s
                   int64_t M, int64_t N, int64_t K, void* stream);
 
 /* The output tile gwa_w8a8_gemm uses for this shape (GWA_W8A8_TILE_*; -1 for
- * an empty shape): 256 x 256 tiles (direct-to-LDS copies, 512 threads; K a
- * multiple of 128) when their rounds over the CUs finish before those of
- * 128 x 128 tiles, else 128 x 128. No reference counterpart: torch._scaled_mm
- * picks its own kernel. */
-enum { GWA_W8A8_TILE_128x128 = 0, GWA_W8A8_TILE_256x256 = 1 };
+ * an empty shape): of 256 x 256 (512 threads; K a multiple of 128 below 2^23),
+ * 128 x 128, 64 (m) x 128 and 64 x 64, the one whose workgroups finish first.
+ * All copy their stages straight to LDS. No reference counterpart:
+ * torch._scaled_mm picks its own kernel. */
+enum { GWA_W8A8_TILE_128x128 = 0, GWA_W8A8_TILE_256x256 = 1, GWA_W8A8_TILE_64x64 = 2, GWA_W8A8_TILE_64x128 = 3 };
 int gwa_w8a8_gemm_tile(int64_t M, int64_t N, int64_t K);
 
 /* Test and tuning hook: every later gwa_w8a8_gemm uses this tile (-1
- * restores the choice above; K % 128 != 0 or K >= 2^23 always takes
- * 128 x 128). Process-wide; returns the previous setting. */
+ * restores the choice above; a forced 256 x 256 takes 128 x 128 where
+ * K % 128 != 0 or K >= 2^23). Process-wide; returns the previous setting. */
 int gwa_w8a8_gemm_force_tile(int tile);
 
 /* AWQ W4A16 linear (the M = 1 adaLN modulation layers).

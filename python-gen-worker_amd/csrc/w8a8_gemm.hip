@@ -5,159 +5,212 @@
 // applies as two further bf16 ops; here they are fused in fp32).
 //
 // Same orientation as the W4A4 kernel: A operand = weight rows (n), B operand
-// = activation rows (m); a 32 x 32 accumulator block D[n][m] holds m = l % 32
-// and n = 8*(v/4) + 4*(l/32) + (v%4) in lane l, a 16 x 16 one m = l % 16 and
-// n = 4*(l/16) + v.
+// = activation rows (m); lane l of a 16 x 16 accumulator block D[n][m] holds
+// m = l % 16 and n = 4*(l/16) + v.
 #include <atomic>
 
 #include "fp6_gemm_common.h"
 
 namespace {
 
-constexpr int TILE = 128;
-constexpr int KT = 128;                 // int8 bytes (= K elements) per row per stage
-constexpr int LDS_STRIDE = KT + 16;
-constexpr int LDS_TILE = TILE * LDS_STRIDE;
-constexpr int LOADS = TILE * KT / 16 / 256;
-constexpr int OSTR = TILE * 2 + 8;     // output staging row: 8-byte pad
-static_assert(TILE * OSTR <= 2 * LDS_TILE, "output staging fits the weight buffers");
+// s_waitcnt lgkmcnt(0), vmcnt and expcnt left at their maxima
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
-template <int BIAS_DT, bool OUT_F16>  // BIAS_DT: -1 none, else GWA_DT_*
-__global__ __launch_bounds__(256) void w8a8_gemm_kernel(const int8_t* __restrict__ qa,
-                                                        const int8_t* __restrict__ qw,
-                                                        const float* __restrict__ sa,
-                                                        const float* __restrict__ sw,
-                                                        const void* __restrict__ bias,
-                                                        uint16_t* __restrict__ out, int M, int N, int K,
-                                                        int sa_row) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds_w[2][LDS_TILE];
-  __shared__ __attribute__((aligned(16))) uint8_t lds_x[2][LDS_TILE];
-  __shared__ __attribute__((aligned(16))) float g_epi[2 * TILE];  // the tile's sw, then its bias as fp32
+template <int BIAS_DT>
+__device__ __forceinline__ float bias_at(const void* bias, int n) {
+  if (BIAS_DT == GWA_DT_F32) return ((const float*)bias)[n];
+  if (BIAS_DT == GWA_DT_BF16) return bf16_to_f32(((const uint16_t*)bias)[n]);
+  if (BIAS_DT == GWA_DT_F16) return f16_bits_to_f32(((const uint16_t*)bias)[n]);
+  return 0.0f;
+}
 
-  const int tiles_n = (N + TILE - 1) / TILE;
-  const int tn = blockIdx.x % tiles_n, tm = blockIdx.x / tiles_n;
-  const int n0 = tn * TILE, m0 = tm * TILE;
-  const int nstages = (K + KT - 1) / KT;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wn = wave & 1, wm = wave >> 1;
-  const int r32 = lane & 31, h = lane >> 5;
-  const int t = threadIdx.x;
+// LDS slot of 16-byte chunk c of operand row r: c ^ l_swz(r), so the 16 rows a quarter of a read instruction
+// touches fill all banks
+__device__ __forceinline__ int l_swz(int r) { return (r >> 1) & 7; }
 
-  v16i acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = (v16i){};
+// Direct-to-LDS copy of 16 bytes per lane at 64-bit lane addresses: LDS [lds_addr + 16 lane, +16) <- src. Every
+// lane's source must be readable; waits are the kernel's (as for dma16).
+__device__ __forceinline__ void dma16_at(uint32_t lds_addr, const uint8_t* src) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(src) : "memory", "m0");
+}
 
-  v4i rw[LOADS], rx[LOADS];
-  auto load = [&](int stage) {
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j) {
-      const int idx = t + j * 256;
-      const int row = idx / (KT / 16), c = idx % (KT / 16);
-      const int kb = stage * KT + c * 16;
-      const bool kin = kb < K;
-      rw[j] = (n0 + row < N && kin) ? *(const v4i*)(qw + (int64_t)(n0 + row) * K + kb) : (v4i){0, 0, 0, 0};
-      rx[j] = (m0 + row < M && kin) ? *(const v4i*)(qa + (int64_t)(m0 + row) * K + kb) : (v4i){0, 0, 0, 0};
+// wait until at most min(newer, most) stages of `copies` copies each are still in flight (and no LDS read)
+template <int copies, int most>
+__device__ __forceinline__ void wait_newer(int newer) {
+  if constexpr (most > 0) {
+    if (newer < most) {
+      wait_newer<copies, most - 1>(newer);
+      return;
     }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j) {
-      const int idx = t + j * 256;
-      const int row = idx / (KT / 16), c = idx % (KT / 16);
-      *(v4i*)(lds_w[buf] + row * LDS_STRIDE + c * 16) = rw[j];
-      *(v4i*)(lds_x[buf] + row * LDS_STRIDE + c * 16) = rx[j];
-    }
-  };
-
-  load(0);
-  if (t < TILE) {  // the epilogue's per-column constants (published by the next barrier)
-    const int n = n0 + t;
-    float wv = 0.0f, bv = 0.0f;
-    if (n < N) {
-      wv = sw[n];
-      if (BIAS_DT == GWA_DT_F32) bv = ((const float*)bias)[n];
-      if (BIAS_DT == GWA_DT_BF16) bv = bf16_to_f32(((const uint16_t*)bias)[n]);
-      if (BIAS_DT == GWA_DT_F16) bv = f16_bits_to_f32(((const uint16_t*)bias)[n]);
-    }
-    g_epi[t] = wv;
-    g_epi[TILE + t] = bv;
   }
-  store(0);
+  wait_vm_lgkm0<copies * most>();
+}
+
+// ---------------------------------------------------------------------------
+// TM x TN tiles (64 or 128) for grids that leave CUs idle on 256 x 256 ones, 4 waves as a 2 x 2 grid. What
+// bounds them is the serial chain of a stage (wait, barrier, operand reads, MFMAs), not bytes: 64 x 64 tiles
+// at K = 12288 take 0.27 us a stage with one workgroup on a CU, and a deeper ring changes nothing (3, 4 and 8
+// buffers: 8.5, 9.0 and 9.4 us at 256 x 3072 x 3072). So the stages are copied straight to LDS (the
+// register-staged form took 22.3 us there on 128 x 128 tiles), each stage's operands are read one stage ahead under
+// the MFMAs (11.4 us without), and the ring is as short as lets several workgroups share a CU and fill each
+// other's gaps.
+// ---------------------------------------------------------------------------
+constexpr int S_KS = 128;  // K bytes per row and stage; K % 128 == 64 ends in half a stage (one k-step)
+
+template <int TM, int TN, int NBUF, int BIAS_DT, bool OUT_F16>
+__global__ __launch_bounds__(256) void w8a8_gemm_small_kernel(const int8_t* __restrict__ qa,
+                                                              const int8_t* __restrict__ qw,
+                                                              const float* __restrict__ sa,
+                                                              const float* __restrict__ sw,
+                                                              const void* __restrict__ bias,
+                                                              uint16_t* __restrict__ out, int M, int N, int K,
+                                                              int sa_row) {
+  constexpr int STAGE = (TM + TN) * S_KS, COPIES = STAGE / 1024 / 4;  // per wave and stage
+  constexpr int BM = TM / 32, BN = TN / 32;                           // 16 x 16 blocks of a wave's half tiles
+  constexpr int OSTR = TN * 2 + 16;
+  static_assert(TM * OSTR <= NBUF * STAGE, "output staging");
+  __shared__ __attribute__((aligned(16))) uint8_t g_lds[NBUF * STAGE];
+  __shared__ __attribute__((aligned(16))) float g_epi[2 * TN];
+  const int tid = threadIdx.x;
+  const int tiles_n = (N + TN - 1) / TN, tiles_m = (M + TM - 1) / TM;
+  int tm, tn;
+  if (!xcd_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;  // whole workgroup, before any barrier
+  const int m0 = tm * TM, n0 = tn * TN;
+  const int nst = (K + S_KS - 1) / S_KS;
+  const bool half = K % S_KS != 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wn = wave & 1, wm = wave >> 1, r16 = lane & 15, q4 = lane >> 4;
+
+  float cs = 0.0f, cb = 0.0f;
+  if (tid < TN && n0 + tid < N) {
+    cs = sw[n0 + tid];
+    cb = bias_at<BIAS_DT>(bias, n0 + tid);
+  }
+  // copy j of this wave is run q = wave + 4 j of a stage: eight rows, lane -> row 8 q + lane / 8, LDS slot
+  // lane % 8; the activation rows first. Rows past M or N re-read the last one (their results are not stored).
+  const uint8_t* src[COPIES];
+  const int chunk = (lane & 7) ^ l_swz((8 * wave + (lane >> 3)) & 15);
+#pragma unroll
+  for (int j = 0; j < COPIES; ++j) {
+    const int row = 8 * (wave + 4 * j) + (lane >> 3);
+    src[j] = 4 * j < TM / 8 ? (const uint8_t*)qa + (int64_t)min(m0 + row, M - 1) * K
+                            : (const uint8_t*)qw + (int64_t)min(n0 + row - TM, N - 1) * K;
+    src[j] += 16 * chunk;
+  }
+  const uint32_t ldst = (uint32_t)(uintptr_t)(g_lds + wave * 1024);
+  auto issue = [&](int u, int st) __attribute__((always_inline)) {
+    // half a stage: the upper chunks (which no k-step reads) come from the lower ones
+    const int back = half && st == nst - 1 && chunk >= 4 ? 64 : 0;
+    int64_t off = (int64_t)st * S_KS - back;
+    if (!GWA_DCHECK(off + 16 * chunk + 16 <= K, kDbgW8Copy, off)) off = 0;
+#pragma unroll
+    for (int j = 0; j < COPIES; ++j) dma16_at(ldst + (uint32_t)(u * STAGE + j * 4096), src[j] + off);
+  };
+
+  v4i acc[BN][BM];
+#pragma unroll
+  for (int bn = 0; bn < BN; ++bn)
+#pragma unroll
+    for (int bm = 0; bm < BM; ++bm) acc[bn][bm] = (v4i){};
+  uint32_t xoff[2], woff[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const uint32_t c = 16u * (uint32_t)((4 * ks + q4) ^ l_swz(r16));
+    xoff[ks] = (uint32_t)((TM / 2 * wm + r16) * S_KS) + c;
+    woff[ks] = (uint32_t)((TM + TN / 2 * wn + r16) * S_KS) + c;
+  }
+
+  // the operands of a stage are read one stage ahead into the other register set, under this stage's MFMAs
+  v4i a[2][2][BN], b[2][2][BM];
+  auto read_ops = [&](int set, int u) __attribute__((always_inline)) {
+    const uint8_t* buf = g_lds + u * STAGE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int bm = 0; bm < BM; ++bm) b[set][ks][bm] = *(const v4i*)(buf + xoff[ks] + bm * 16 * S_KS);
+#pragma unroll
+      for (int bn = 0; bn < BN; ++bn) a[set][ks][bn] = *(const v4i*)(buf + woff[ks] + bn * 16 * S_KS);
+    }
+  };
+  auto mma = [&](int set, int ks) __attribute__((always_inline)) {
+#pragma unroll
+    for (int bn = 0; bn < BN; ++bn)
+#pragma unroll
+      for (int bm = 0; bm < BM; ++bm)
+        acc[bn][bm] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[set][ks][bn], b[set][ks][bm], acc[bn][bm], 0, 0, 0);
+  };
+#pragma unroll
+  for (int st = 0; st < NBUF; ++st)
+    if (st < nst) issue(st, st);
+  wait_newer<COPIES, NBUF - 1>(min(NBUF - 1, nst - 1));
+  barrier_lds();
+  read_ops(0, 0);
+  int u = 0;  // buffer of stage st
+  auto stage = [&](int set, int st) __attribute__((always_inline)) {
+    const int v = u == NBUF - 1 ? 0 : u + 1;
+    if (st + 1 < nst) {
+      wait_newer<COPIES, NBUF - 2>(min(NBUF - 2, nst - 2 - st));
+      barrier_lds();  // everyone's copies of stage st + 1 are in, and everyone's reads of stage st have ended
+      read_ops(set ^ 1, v);
+      if (st + NBUF < nst) issue(u, st + NBUF);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mma(set, 0);
+    if (!(half && st == nst - 1)) mma(set, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    u = v;
+  };
+  for (int st = 0; st < nst; st += 2) {
+    stage(0, st);
+    if (st + 1 < nst) stage(1, st + 1);
+  }
+
+  // epilogue: y = acc * sa[m] * sw[n] + bias[n], staged as [m][n] rows and stored as whole row segments
+  if (tid < TN) {
+    g_epi[tid] = cs;
+    g_epi[TN + tid] = cb;
+  }
   __syncthreads();
-  for (int st = 0; st < nstages; ++st) {
-    const int buf = st & 1;
-    if (st + 1 < nstages) load(st + 1);
-    const uint8_t* lw = lds_w[buf];
-    const uint8_t* lx = lds_x[buf];
 #pragma unroll
-    for (int ks = 0; ks < KT / 32; ++ks) {
-      v4i a[2], b[2];
+  for (int bm = 0; bm < BM; ++bm) {
+    const int ml = TM / 2 * wm + 16 * bm + r16;
+    const float am = sa[sa_row ? min(m0 + ml, M - 1) : 0];  // rows past M are computed but never stored
 #pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-        a[bn] = *(const v4i*)(lw + (64 * wn + 32 * bn + r32) * LDS_STRIDE + ks * 32 + 16 * h);
+    for (int bn = 0; bn < BN; ++bn) {
+      const int nl = TN / 2 * wn + 16 * bn + 4 * q4;
+      const v4f cw = *(const v4f*)(g_epi + nl);
+      const v4f cv = *(const v4f*)(g_epi + TN + nl);
+      float o[4];
 #pragma unroll
-      for (int bm = 0; bm < 2; ++bm)
-        b[bm] = *(const v4i*)(lx + (64 * wm + 32 * bm + r32) * LDS_STRIDE + ks * 32 + 16 * h);
-#pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < 2; ++bm)
-          acc[bn][bm] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[bn], b[bm], acc[bn][bm], 0, 0, 0);
-    }
-    if (st + 1 < nstages) store(buf ^ 1);
-    __syncthreads();
-  }
-
-  // epilogue as in the 256 x 256 kernel: constants from LDS, the packed tile staged in the (free) weight
-  // buffers as [m][n] rows, stored as whole row segments
-  uint8_t* ob = lds_w[0];
-#pragma unroll
-  for (int bm = 0; bm < 2; ++bm) {
-    const int ml = 64 * wm + 32 * bm + r32, m = m0 + ml;
-    const float am = sa[sa_row ? min(m, M - 1) : 0];  // rows past M are computed but never stored
-#pragma unroll
-    for (int bn = 0; bn < 2; ++bn) {
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int nl = 64 * wn + 32 * bn + 8 * qd + 4 * h;
-        if (n0 + nl >= N) continue;  // N % 16 == 0: n < N covers n + 3
-        const v4f cw = *(const v4f*)(g_epi + nl);
-        const v4f cb = *(const v4f*)(g_epi + TILE + nl);
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float y = (float)acc[bn][bm][4 * qd + e] * am * cw[e];
-          if (BIAS_DT >= 0) y += cb[e];
-          o[e] = y;
-        }
-        uint2 pk;
-        if (OUT_F16) {
-          pk.x = pack_f16x2(o[0], o[1]);
-          pk.y = pack_f16x2(o[2], o[3]);
-        } else {
-          pk.x = pack_bf16x2_rn(o[0], o[1]);
-          pk.y = pack_bf16x2_rn(o[2], o[3]);
-        }
-        *(uint2*)(ob + ml * OSTR + nl * 2) = pk;
+      for (int e = 0; e < 4; ++e) {
+        float y = (float)acc[bn][bm][e] * am * cw[e];
+        if (BIAS_DT >= 0) y += cv[e];
+        o[e] = y;
       }
+      uint2 pk;
+      if (OUT_F16) {
+        pk.x = pack_f16x2(o[0], o[1]);
+        pk.y = pack_f16x2(o[2], o[3]);
+      } else {
+        pk.x = pack_bf16x2_rn(o[0], o[1]);
+        pk.y = pack_bf16x2_rn(o[2], o[3]);
+      }
+      *(uint2*)(g_lds + ml * OSTR + nl * 2) = pk;
     }
   }
   __syncthreads();
   // a descriptor over this tile's output span (127 N + 128 elements < 2^28: N < 2^21 is checked on the host)
-  const int rows = min(M - m0, TILE), cols = min(N - n0, TILE);
-  const rsrc_t obuf = make_rsrc(out + (int64_t)m0 * N + n0, (uint32_t)(((rows - 1) * N + cols) * 2));
-  constexpr int CPR = TILE / 8;  // 16-byte chunks per row
-#pragma unroll 4
-  for (int i = t; i < TILE * CPR; i += 256) {
+  const int rows = min(M - m0, TM), cols = min(N - n0, TN);
+  const uint32_t span = (uint32_t)(((rows - 1) * N + cols) * 2);
+  const rsrc_t obuf = make_rsrc(out + (int64_t)m0 * N + n0, span);
+  constexpr int CPR = TN / 8;  // 16-byte chunks per row
+#pragma unroll
+  for (int i = tid; i < TM * CPR; i += 256) {
     const int row = i / CPR, c = i % CPR;
-    const uint2 lo = *(const uint2*)(ob + row * OSTR + c * 16);
-    const uint2 hi = *(const uint2*)(ob + row * OSTR + c * 16 + 8);
+    const v4i v = *(const v4i*)(g_lds + row * OSTR + c * 16);
     uint32_t off = row < rows && 8 * c < cols ? (uint32_t)((row * N + 8 * c) * 2) : kOOB;
-    if (!GWA_DCHECK(off == kOOB || (int64_t)off + 16 <= (int64_t)((rows - 1) * N + cols) * 2, kDbgW8Out, off))
-      off = kOOB;
-    buf_store16((v4i){(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y}, obuf, off);
+    if (!GWA_DCHECK(off == kOOB || (int64_t)off + 16 <= (int64_t)span, kDbgW8Out, off)) off = kOOB;
+    buf_store16(v, obuf, off);
   }
 }
 
@@ -195,11 +248,6 @@ constexpr int L_SLOTS = L_STAGE / 1024 / NWAVES;   // copies per wave and stage:
 constexpr int L_LDS = 2 * L_STAGE;
 static_assert(L_LDS <= kLdsBytes && L_SLOTS * NWAVES * 1024 == L_STAGE, "stage layout");
 static_assert(NWAVES * 64 * 256 <= L_LDS, "output staging");
-
-__device__ __forceinline__ int l_swz(int r) { return (r >> 1) & 7; }
-
-// s_waitcnt lgkmcnt(0), vmcnt and expcnt left at their maxima
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
 template <int BIAS_DT, bool OUT_F16>
 __global__ __launch_bounds__(NTHREADS, 1) void w8a8_gemm_lds_kernel(const int8_t* __restrict__ qa,
@@ -384,24 +432,53 @@ std::atomic<int> g_w8a8_force_tile{-1};  // test / tuning hook (gwa_w8a8_gemm_fo
 using W8Kernel = void (*)(const int8_t*, const int8_t*, const float*, const float*, const void*, uint16_t*, int, int,
                           int, int);
 
-template <int BD>
-W8Kernel pick_kernel(int tile, bool f16) {
-  if (tile == GWA_W8A8_TILE_256x256) return f16 ? w8a8_gemm_lds_kernel<BD, true> : w8a8_gemm_lds_kernel<BD, false>;
-  return f16 ? w8a8_gemm_kernel<BD, true> : w8a8_gemm_kernel<BD, false>;
+// A tile's geometry, the workgroups of it a CU holds at once (LDS), and the time of one to that many of them on a
+// CU at K = 3072, in 0.1 us (measured; 256 x 3072 and 9216, 1024 and 2048 x 3072, 512 and 1024 x 9216).
+struct W8Tile {
+  int tm, tn, held;
+  int us10[3];
+};
+constexpr W8Tile kTiles[] = {{128, 128, 2, {180, 232}}, {256, 256, 1, {335}}, {64, 64, 3, {85, 125, 165}},
+                             {64, 128, 2, {114, 158}}};
+
+template <int BD, bool F16>
+W8Kernel pick_kernel(int tile) {
+  switch (tile) {
+    case GWA_W8A8_TILE_256x256: return w8a8_gemm_lds_kernel<BD, F16>;
+    case GWA_W8A8_TILE_64x64: return w8a8_gemm_small_kernel<64, 64, 3, BD, F16>;
+    case GWA_W8A8_TILE_64x128: return w8a8_gemm_small_kernel<64, 128, 3, BD, F16>;
+    default: return w8a8_gemm_small_kernel<128, 128, 2, BD, F16>;
+  }
 }
 
-// 256 x 256 tiles when their rounds over the CUs finish first: a 256 x 256 tile takes about 2.7 times as
-// long as a 128 x 128 one (four times the work at a higher rate: 50 us against 18.3 us at K = 3072), so the
-// choice compares ceil(tiles / CUs) rounds of each; 128-byte stages need K % 128 == 0, and the per-tile
-// descriptors 256 K < 2^31
+int64_t w8a8_tiles(int tile, int64_t M, int64_t N) {
+  const W8Tile& t = kTiles[tile];
+  return ((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
+}
+
+// The tile that finishes first: the most workgroups a CU gets, in batches of as many as it holds, at the batch
+// times above (they scale with K alike, so their order holds at any K). Measured at the picks against 128 x 128
+// for everything below 256 x 256's grids, register-staged (the form before): 256 x 3072 x 3072 64 x 64 8.5 us
+// (22.3), 256 x 9216 64 x 128 16.1 (24.4), 1024 x 3072 64 x 128 15.5 (24.5), 512 x 9216 128 x 128 22.6 (29.1),
+// 2048 x 3072 128 x 128 23.7 (31.6), K = 12288 at 256 x 3072 64 x 64 26.7 (83.6). 256 x 256's stages need
+// K % 128 == 0 and its descriptors 256 K < 2^31.
 int w8a8_tile(int64_t M, int64_t N, int64_t K) {
-  if (K % L_KS || K >= (1ll << 23)) return GWA_W8A8_TILE_128x128;
+  const bool big_ok = K % L_KS == 0 && K < (1ll << 23);
   const int forced = g_w8a8_force_tile.load(std::memory_order_relaxed);
-  if (forced >= 0) return forced;
-  const int64_t big = ((M + L_TM - 1) / L_TM) * ((N + L_TN - 1) / L_TN);
-  const int64_t small = ((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
-  const int64_t rounds_big = (big + kCus - 1) / kCus, rounds_small = (small + kCus - 1) / kCus;
-  return 27 * rounds_big < 10 * rounds_small ? GWA_W8A8_TILE_256x256 : GWA_W8A8_TILE_128x128;
+  if (forced >= 0) return forced == GWA_W8A8_TILE_256x256 && !big_ok ? GWA_W8A8_TILE_128x128 : forced;
+  int best = -1;
+  int64_t best_us = 0;
+  for (int t = 0; t < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++t) {
+    if (t == GWA_W8A8_TILE_256x256 && !big_ok) continue;
+    const int64_t per_cu = (w8a8_tiles(t, M, N) + kCus - 1) / kCus, held = kTiles[t].held;
+    int64_t us = per_cu / held * kTiles[t].us10[held - 1];
+    if (per_cu % held) us += kTiles[t].us10[per_cu % held - 1];
+    if (best < 0 || us < best_us) {
+      best = t;
+      best_us = us;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -412,7 +489,7 @@ extern "C" int gwa_w8a8_gemm_tile(int64_t M, int64_t N, int64_t K) {
 }
 
 extern "C" int gwa_w8a8_gemm_force_tile(int tile) {
-  return g_w8a8_force_tile.exchange(tile == GWA_W8A8_TILE_128x128 || tile == GWA_W8A8_TILE_256x256 ? tile : -1);
+  return g_w8a8_force_tile.exchange(tile >= 0 && tile <= GWA_W8A8_TILE_64x128 ? tile : -1);
 }
 
 extern "C" int gwa_w8a8_gemm(const int8_t* qa, const int8_t* qw, const float* sa, int64_t sa_numel,
@@ -434,23 +511,22 @@ extern "C" int gwa_w8a8_gemm(const int8_t* qa, const int8_t* qw, const float* sa
   GWA_REQUIRE(GWA_ALIGNED(qa, 16) && GWA_ALIGNED(qw, 16) && GWA_ALIGNED(out, 8) && GWA_ALIGNED(sa, 4) &&
                   GWA_ALIGNED(sw, 4) && GWA_ALIGNED(bias, 2),
               "w8a8_gemm: qa/qw must be 16-byte and out 8-byte aligned");
-  const int64_t tiles = ((M + TILE - 1) / TILE) * ((N + TILE - 1) / TILE);
-  GWA_REQUIRE(tiles < (1ll << 31), "w8a8_gemm: too many tiles");
+  const int tile = w8a8_tile(M, N, K);
+  const int64_t tiles = w8a8_tiles(tile, M, N);
+  GWA_REQUIRE(tiles < (1ll << 31) - kXcds && w8a8_tiles(GWA_W8A8_TILE_128x128, M, N) < (1ll << 31),
+              "w8a8_gemm: too many tiles");
   hipStream_t s = (hipStream_t)stream;
   const bool f16 = out_dtype == GWA_DT_F16;
   uint16_t* op = (uint16_t*)out;
   const int m = (int)M, n = (int)N, k = (int)K, sr = sa_numel == M && M > 1 ? 1 : 0;
-  const int tile = w8a8_tile(M, N, K);
-  const bool lds = tile != GWA_W8A8_TILE_128x128;
-  const int64_t big = ((M + L_TM - 1) / L_TM) * ((N + L_TN - 1) / L_TN);
-  const int64_t per_xcd = (big + kXcds - 1) / kXcds;
-  const dim3 grid(lds ? (unsigned)(per_xcd * kXcds) : (unsigned)tiles), block(lds ? NTHREADS : 256);
+  const dim3 grid((unsigned)((tiles + kXcds - 1) / kXcds * kXcds));
+  const dim3 block(tile == GWA_W8A8_TILE_256x256 ? NTHREADS : 256);
   const int bd = bias ? bias_dtype : -1;
   W8Kernel kern = nullptr;
-  if (bd == -1) kern = pick_kernel<-1>(tile, f16);
-  else if (bd == GWA_DT_F32) kern = pick_kernel<GWA_DT_F32>(tile, f16);
-  else if (bd == GWA_DT_BF16) kern = pick_kernel<GWA_DT_BF16>(tile, f16);
-  else kern = pick_kernel<GWA_DT_F16>(tile, f16);
+  if (bd == -1) kern = f16 ? pick_kernel<-1, true>(tile) : pick_kernel<-1, false>(tile);
+  else if (bd == GWA_DT_F32) kern = f16 ? pick_kernel<GWA_DT_F32, true>(tile) : pick_kernel<GWA_DT_F32, false>(tile);
+  else if (bd == GWA_DT_BF16) kern = f16 ? pick_kernel<GWA_DT_BF16, true>(tile) : pick_kernel<GWA_DT_BF16, false>(tile);
+  else kern = f16 ? pick_kernel<GWA_DT_F16, true>(tile) : pick_kernel<GWA_DT_F16, false>(tile);
   hipLaunchKernelGGL(kern, grid, block, 0, s, qa, qw, sa, sw, bias, op, m, n, k, sr);
   return gwa_check_launch("w8a8_gemm");
 }

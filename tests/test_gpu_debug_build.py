@@ -113,7 +113,7 @@ def test_debug_build_w8a8_no_violation_and_identical(libs, m, n, k):
     outs = {}
     for name, lib in (("rel", rel), ("dbg", dbg)):
         res = []
-        for tile in (0, 1):
+        for tile in range(4):
             lib.gwa_w8a8_gemm_force_tile(tile)
             out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
             _ok(lib.gwa_w8a8_gemm(qa.data_ptr(), qw.data_ptr(), sa.data_ptr(), m, sw.data_ptr(), bias.data_ptr(), 0,

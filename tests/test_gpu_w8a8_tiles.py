@@ -1,8 +1,7 @@
 """GPU coverage of every output tile of the W8A8 GEMM (``gwa_w8a8_gemm``).
 
-The GEMM picks 256 x 256 tiles (direct-to-LDS copies, eight waves; stages of 64 or 128 K-bytes) when they
-give every CU a tile, else 128 x 128 (register-staged copies); ``gwa_w8a8_gemm_force_tile`` pins one. All
-accumulate the exact int32 dot product and apply the same fp32 epilogue, so their outputs must agree bit for
+The GEMM picks the one of its 256 x 256, 128 x 128, 64 x 128 and 64 x 64 tiles whose workgroups finish first;
+``gwa_w8a8_gemm_force_tile`` pins one. All accumulate the exact int32 dot product and apply the same fp32 epilogue, so their outputs must agree bit for
 bit on ragged shapes,
 short K (one to three stages, fewer than the copy pipeline's depth), both scale modes, every bias dtype and
 both output dtypes; each is also checked against the oracle's float64 linear (``oracle/svdq_oracle.py``
@@ -116,3 +115,22 @@ def test_large_shapes_take_the_large_tile_and_agree(force):
     acc = qa[rows].double() @ qw.double().t()
     ref = (acc.float() * sa[rows, None] * sw[None, :] + bias[None, :]).double().cpu().numpy()
     check_output(y[rows], ref, what="w8a8 QKV 4608")
+
+
+# tile edges and remainders of the 64-row tiles; K of half a stage, one stage, fewer stages than the copy ring's
+# three buffers, exactly that many, and more, with and without a half stage at the end
+@pytest.mark.parametrize("m,n,k,pertensor,bdt,odt", [
+    (1, 16, 64, False, torch.float32, torch.bfloat16), (64, 64, 128, False, None, torch.bfloat16),
+    (65, 80, 192, True, torch.bfloat16, torch.float16), (63, 272, 384, False, torch.float16, torch.bfloat16),
+    (129, 144, 448, False, torch.float32, torch.float16), (200, 400, 1088, True, torch.float32, torch.bfloat16)])
+def test_small_tiles_agree_and_match_oracle(force, m, n, k, pertensor, bdt, odt):
+    xb, qa, sa, qw, sw, b = _operands(m, n, k, seed=m + n + k, pertensor=pertensor)
+    bias = _bias(b, bdt)
+    outs = []
+    for tile in (SMALL, 2, 3):  # 128 x 128, GWA_W8A8_TILE_64x64, GWA_W8A8_TILE_64x128
+        force(tile)
+        outs.append(_run(qa, sa, qw, sw, bias, odt))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, outs[0]) for o in outs), f"tiles differ at {(m, n, k)}"
+    bref = None if bdt is None else bias.float().cpu().numpy()
+    check_output(outs[1], O.w8a8_linear(xb, qw, sw, bref, pertensor=pertensor), what=f"w8a8 64x64 tile {(m, n, k)}")
