@@ -168,6 +168,13 @@ def load() -> ctypes.CDLL:
                 raise NativeUnavailable(f"{path} does not export {name}")
             fn.argtypes = list(argtypes)
             fn.restype = _RESTYPES.get(name, ctypes.c_int)
+        try:
+            from . import ops
+
+            ops.bind_host_calls(lib)
+        except ImportError as exc:
+            raise NativeUnavailable(f"the native host calls failed to load (build them with `python -m "
+                                    f"gen_worker_amd.build`): {exc}") from exc
         _lib = lib
         return lib
 

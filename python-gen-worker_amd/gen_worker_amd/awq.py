@@ -39,6 +39,8 @@ import torch
 import torch.nn as nn
 from torch import Tensor
 
+from . import ops
+
 GROUP_SIZE = 64
 _SCALE_PACK = 8                     # scale rows are written in packs of 8 groups
 _PACK_MULTIPLE = {32: 4, 64: 2}     # and the pack count rounded up to this multiple per group size
@@ -340,6 +342,12 @@ class AwqPackedLinear(nn.Module):
         return mod
 
     def forward(self, x: Tensor) -> Tensor:
+        native = ops.awq_native()
+        if native is not None and not torch.compiler.is_compiling():
+            b = self._buffers
+            y = native(x, b["weight"], b["wscales"], b["wzeros"], self.bias, ops.AWQ_GEMV_MAX_M)
+            if y is not None:
+                return y
         lead = x.shape[:-1]
         y = torch.ops.cozy_gen_worker.awq_w4a16_mm(x.reshape(-1, self.in_features).contiguous(), self.weight,
                                                    self.wscales, self.wzeros, self.bias)

@@ -1,6 +1,7 @@
-"""Build the C-ABI library ``libgen_worker_amd.so`` for gfx950 with hipcc.
+"""Build the C-ABI library ``libgen_worker_amd.so`` for gfx950 with hipcc, and the native host calls
+(``_host_calls``, a CPython extension on torch's headers) with the host compiler.
 
-The library is built in-tree (next to this file) so that it travels with the
+Both are built in-tree (next to this file) so that they travel with the
 source tree; nothing is installed. ``python -m gen_worker_amd.build`` or
 ``__graft_entry__.build()`` runs it.
 """
@@ -12,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -22,6 +24,8 @@ LIB_NAME = "libgen_worker_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 DEBUG_LIB_NAME = "libgen_worker_amd_debug.so"
 DEBUG_LIB_PATH = PKG_DIR / DEBUG_LIB_NAME
+HOST_CALLS_SRC = "host_calls.cpp"
+HOST_CALLS_PATH = PKG_DIR / ("_host_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 ARCH = "gfx950"
 
 SOURCES = ("gwa_runtime.hip", "act_quant.hip", "w4a4_gemm.hip", "w4a4_gemm_fp6.hip", "w4a4_gemm_fp6_pipe.hip",
@@ -72,16 +76,38 @@ def _build_one(debug: bool, ex: cf.Executor) -> Path:
     return lib_path
 
 
+def _build_host_calls() -> Path:
+    """Compile and link the native host calls against the installed torch; returns the extension's path."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    tmp = HOST_CALLS_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{d}" for d in include_paths()), "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+           f"-I{INCLUDE}", str(CSRC / HOST_CALLS_SRC), f"-L{lib_dir}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+           "-ltorch_hip", "-ltorch_python", "-o", str(tmp)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{HOST_CALLS_SRC} failed to build:\n{res.stderr[-6000:]}")
+    os.replace(tmp, HOST_CALLS_PATH)
+    return HOST_CALLS_PATH
+
+
 def build(verbose: bool = False, jobs: int | None = None, debug: bool = True) -> Path:
-    """Compile every HIP source for gfx950 and link the shared library; returns its path. With ``debug`` the
+    """Compile every HIP source for gfx950 and link the shared library, and build the native host calls; returns the
+    library's path. With ``debug`` the
     same sources are also built with GWA_DEBUG (device-side bounds checks that record violations, read with
     ``gwa_debug_violations``) into ``libgen_worker_amd_debug.so``."""
     jobs = jobs or max(1, (os.cpu_count() or 2) - 1)
-    # the two builds wait on compile jobs of a pool of their own, so neither can starve the other
-    with cf.ThreadPoolExecutor(max_workers=jobs) as cex, cf.ThreadPoolExecutor(max_workers=2) as bex:
+    # the library builds wait on compile jobs of a pool of their own, so neither can starve the other
+    with cf.ThreadPoolExecutor(max_workers=jobs) as cex, cf.ThreadPoolExecutor(max_workers=3) as bex:
+        host = bex.submit(_build_host_calls)
         rel = bex.submit(_build_one, False, cex)
         dbg = bex.submit(_build_one, True, cex) if debug else None
         path = rel.result()
+        host.result()
         if dbg is not None:
             dpath = dbg.result()
             if verbose:

@@ -144,14 +144,18 @@ def _quant_impl(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor],
     return q, s, la
 
 
-@torch.library.custom_op("cozy_gen_worker::svdq_quant", mutates_args=())
-def svdq_quant(x2: Tensor, smooth: Optional[Tensor], s2: Tensor, blocked: bool) -> tuple[Tensor, Tensor]:
-    """int4 group-64 activation quant: (packed codes uint8 [M, K/2], fp16 scales [M, K/64])."""
+def _svdq_quant_body(x2: Tensor, smooth: Optional[Tensor], s2: Tensor, blocked: bool) -> tuple[Tensor, Tensor]:
     if blocked:
         raise SvdqOpError("svdq_quant: int4 group scales are flat [M, K/64]; the blocked (cuBLAS 128x4 "
                           "tile) layout is an nvfp4 format and is not produced")
     q, s, _ = _quant_impl(x2, smooth, s2, None)
     return q, s
+
+
+@torch.library.custom_op("cozy_gen_worker::svdq_quant", mutates_args=())
+def svdq_quant(x2: Tensor, smooth: Optional[Tensor], s2: Tensor, blocked: bool) -> tuple[Tensor, Tensor]:
+    """int4 group-64 activation quant: (packed codes uint8 [M, K/2], fp16 scales [M, K/64])."""
+    return _svdq_quant_body(x2, smooth, s2, blocked)
 
 
 @svdq_quant.register_fake
@@ -660,6 +664,69 @@ def eager_call_ok(x2: Tensor) -> bool:
             and torch._C._len_torch_dispatch_stack() == 0)
 
 
+def bind_host_calls(lib) -> None:
+    """Give the native host calls (``csrc/host_calls.cpp``) the loaded library's entry points and the Python bodies
+    they hand back to; from then on ``svdq_quant`` and ``svdq_gemm_w4a4_lora`` run their native CUDA kernels."""
+    import ctypes
+
+    from . import _host_calls
+
+    addresses = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in nat.EXPORTED_SYMBOLS}
+    bodies = {"svdq_quant": _svdq_quant_body, "svdq_gemm_w4a4_lora": _svdq_gemm_w4a4_lora_body}
+    _host_calls.bind(addresses, bodies, _REF_WEIGHT_FP6.get)
+    global _awq_native
+    _awq_native = _host_calls.awq_forward
+
+
+_awq_native = None   # the AWQ layer's native call, once the library is loaded
+
+
+def awq_native():
+    """``(x, weight, wscales, wzeros, bias, max_rows) -> output``, or None where ``awq_w4a16_mm`` has to decide (every
+    operand is checked on each call); None before the library is loaded."""
+    return _awq_native
+
+
+def _native_call(kind: int, mod, names: tuple, operands: tuple, versions: tuple, out_dtype: torch.dtype, k: int,
+                 n: int, rank: int, gemv_max_m: int, flags: int):
+    """A native bound call for ``mod``: good while each of ``names`` is the object it is now and each operand keeps
+    its storage (and version, where one is given); None for a module that keeps one of them elsewhere."""
+    from . import _host_calls
+
+    attrs = []
+    for name in names:
+        for where, d in enumerate((mod.__dict__, mod._buffers, mod._parameters)):
+            if name in d:
+                attrs.append((where, name, d[name]))
+                break
+        else:
+            return None
+    return _host_calls.BoundCall(kind, attrs, list(operands), list(versions), out_dtype, k, n, rank, gemv_max_m, flags)
+
+
+def native_w4a4(mod, out_dtype: torch.dtype, gelu: bool):
+    """The native bound call of a ``SvdqW4A4Linear`` in the fp6 lane."""
+    names = ("weight_fp6", "weight", "weight_scale", "smooth_factor", "proj_down", "proj_down_op6", "proj_up", "second",
+             "bias", "out_dtype", "activation", "rank", "in_features", "out_features", "_gemv_max_m", "_derived_from")
+    from_versions = tuple(None if v is None else v[1] for v in mod._derived_from)
+    return _native_call(0, mod, names, (mod.weight_fp6, mod.smooth_factor, mod.proj_down_op6 if mod.rank else None,
+                                        mod.weight, mod.weight_scale, mod.second, mod.proj_up if mod.rank else None,
+                                        mod.bias, mod.proj_down if mod.rank else None),
+                        (None, None, None, from_versions[0], from_versions[1], None, None, None, from_versions[2]),
+                        out_dtype, mod.in_features, mod.out_features, mod.rank, mod._gemv_max_m,
+                        nat.EPI_GELU_TANH if gelu else 0)
+
+
+def native_w8a8(mod):
+    """The native bound call of an ``Int8ScaledLinear`` (None with a LoRA addend, which its forward adds)."""
+    if mod.lora_a is not None:
+        return None
+    names = ("weight", "weight_scale", "bias", "input_scale", "gemm_mode", "compute_dtype", "lora_a", "in_features",
+             "out_features")
+    return _native_call(1, mod, names, (mod.weight, mod.weight_scale, mod.bias, mod.input_scale), (None,) * 4,
+                        mod.compute_dtype, mod.in_features, mod.out_features, 0, 0, int(mod.gemm_mode == "pertensor"))
+
+
 class BoundLinearFp6:
     """One fp6-lane linear's resident operands bound for eager calls: the same library entry points and
     arguments as ``svdq_forward_fp6`` (and ``svdq_forward_gemv`` up to ``gemv_max_m`` tokens), so the output is
@@ -667,9 +734,10 @@ class BoundLinearFp6:
     checked once, by running both ops on a 0-row activation; a call then checks only the activation (dtype,
     device, width; rows with an unaligned stride are copied, as the op does), allocates the output and the
     workspace and enqueues on the current stream. The pointers are those of the tensors at binding: the owner
-    rebinds when any of them changes (``key``), and the binding holds them (``held``)."""
+    rebinds when any of them changes (``key``), and the binding holds them (``held``). ``native`` is the same call
+    in native code, which the owner tries first."""
 
-    __slots__ = ("key", "held", "device", "k", "n", "rank", "out_dtype", "gemv_max_m", "_lin", "_gemv",
+    __slots__ = ("key", "held", "native", "device", "k", "n", "rank", "out_dtype", "gemv_max_m", "_lin", "_gemv",
                  "_lin_args", "_gemv_args", "_tail", "_ws_lin", "_ws_gemv", "_ws", "_dev_index")
 
     def __init__(self, *, key: tuple, held: tuple, k: int, smooth: Optional[Tensor], proj_down_op6: Optional[Tensor],
@@ -686,6 +754,7 @@ class BoundLinearFp6:
             raise SvdqOpError("BoundLinearFp6: second must be float32 (the op would convert it per call)")
         lib = nat.load()
         self.key = key
+        self.native = None
         self.held = held  # the bound pointers' tensors stay allocated while the binding exists
         self.device = weight_fp6.device
         self._dev_index = self.device.index if self.device.index is not None else torch.cuda.current_device()
@@ -920,14 +989,8 @@ def reference_gemm_weight_cache() -> _Fp6WeightCache:
     return _REF_WEIGHT_FP6
 
 
-@torch.library.custom_op("cozy_gen_worker::svdq_gemm_w4a4_lora", mutates_args=())
-def svdq_gemm_w4a4_lora(qa: Tensor, sa: Tensor, wq_kn: Tensor, ws: Tensor, s2: Tensor, second: Tensor,
-                        lora_act: Tensor, up: Tensor, bias: Optional[Tensor]) -> Tensor:
-    """The reference schema (``models/svdq_fused.py:379-389``): int4 nibble activations ``qa`` [M, K/2] with
-    fp16 scales ``sa`` [M, K/64], the K-major weight ``wq_kn`` [K/2, N] with ``ws`` [N, K/64], bf16 out.
-    It runs the fp6 lane: the activations repacked as fp6 records each call, the weight's records built once
-    per weight tensor (``reference_gemm_weight_cache``); operands outside that lane's contract (or M == 0) go
-    to the general lane, which raises the contract error."""
+def _svdq_gemm_w4a4_lora_body(qa: Tensor, sa: Tensor, wq_kn: Tensor, ws: Tensor, s2: Tensor, second: Tensor,
+                              lora_act: Tensor, up: Tensor, bias: Optional[Tensor]) -> Tensor:
     name = "svdq_gemm_w4a4_lora"
     _check_cuda(name, wq_kn=wq_kn, qa=qa, sa=sa, ws=ws)
     _check_dtype(name, wq_kn, torch.uint8, what="wq_kn")
@@ -945,6 +1008,17 @@ def svdq_gemm_w4a4_lora(qa: Tensor, sa: Tensor, wq_kn: Tensor, ws: Tensor, s2: T
     w_nk = torch.empty(n, kh, dtype=torch.uint8, device=wq_kn.device)
     nat.call("gwa_transpose_2d", nat.ptr(wq_kn), nat.ptr(w_nk), kh, n, 1, nat.stream_of(wq_kn))
     return _gemm_impl(qa, sa, w_nk, ws, s2, second, lora_act, up, bias, torch.bfloat16, False)
+
+
+@torch.library.custom_op("cozy_gen_worker::svdq_gemm_w4a4_lora", mutates_args=())
+def svdq_gemm_w4a4_lora(qa: Tensor, sa: Tensor, wq_kn: Tensor, ws: Tensor, s2: Tensor, second: Tensor,
+                        lora_act: Tensor, up: Tensor, bias: Optional[Tensor]) -> Tensor:
+    """The reference schema (``models/svdq_fused.py:379-389``): int4 nibble activations ``qa`` [M, K/2] with
+    fp16 scales ``sa`` [M, K/64], the K-major weight ``wq_kn`` [K/2, N] with ``ws`` [N, K/64], bf16 out.
+    It runs the fp6 lane: the activations repacked as fp6 records each call, the weight's records built once
+    per weight tensor (``reference_gemm_weight_cache``); operands outside that lane's contract (or M == 0) go
+    to the general lane, which raises the contract error."""
+    return _svdq_gemm_w4a4_lora_body(qa, sa, wq_kn, ws, s2, second, lora_act, up, bias)
 
 
 @svdq_gemm_w4a4_lora.register_fake
@@ -1071,9 +1145,9 @@ class BoundLinearW8a8:
     and the per-call operand checks. The operands are checked once by both ops on a 0-row activation; a call
     checks the activation (bf16, contiguous [M, K] on this device) and allocates the codes, the activation
     scales and the output. The owner rebinds when an operand changes (``key``); the binding holds the tensors
-    whose pointers it uses (``held``)."""
+    whose pointers it uses (``held``). ``native`` is the same call in native code, which the owner tries first."""
 
-    __slots__ = ("key", "held", "device", "k", "n", "pertensor", "dynamic_pt", "out_dtype", "_quant", "_gemm",
+    __slots__ = ("key", "held", "native", "device", "k", "n", "pertensor", "dynamic_pt", "out_dtype", "_quant", "_gemm",
                  "_q_args", "_g_args", "_dev_index")
 
     def __init__(self, *, key: tuple, held: tuple, weight: Tensor, weight_scale: Tensor, bias: Optional[Tensor],
@@ -1083,7 +1157,7 @@ class BoundLinearW8a8:
         q0, sa0 = w8a8_quant(x0, pertensor, static)
         w8a8_scaled_mm(q0, weight, sa0, weight_scale, bias, out_dtype)
         lib = nat.load()
-        self.key, self.held = key, held
+        self.key, self.held, self.native = key, held, None
         self.device = weight.device
         self._dev_index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         self.k, self.n = k, n

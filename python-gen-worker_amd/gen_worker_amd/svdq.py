@@ -263,6 +263,11 @@ class SvdqW4A4Linear(nn.Module):
             out_dtype or self.out_dtype or torch.bfloat16, self.activation == "gelu_tanh")
 
     def forward(self, x: Tensor) -> Tensor:
+        b = self._bound
+        if b is not None and b.native is not None and not torch.compiler.is_compiling():
+            y = b.native.run(x, self.__dict__)
+            if y is not None:
+                return y
         shape = x.shape
         x2 = self._input2d(x)
         out_dtype = self.out_dtype or torch.bfloat16
@@ -309,6 +314,7 @@ class SvdqW4A4Linear(nn.Module):
                 key=key, held=ts, k=self.in_features, smooth=self.smooth_factor, proj_down_op6=pdo6, weight=self.weight,
                 weight_scale=self.weight_scale, weight_fp6=self.weight_fp6, second=self.second, proj_up=up,
                 bias=self.bias, out_dtype=out_dtype, gelu=gelu, gemv_max_m=self._gemv_max_m)
+            b.native = ops.native_w4a4(self, out_dtype, gelu)
         return b(x2)
 
     def extra_repr(self) -> str:

@@ -85,6 +85,11 @@ class Int8ScaledLinear(nn.Module):
         return (x2 @ self.lora_a.t()) @ self.lora_b.t()
 
     def forward(self, x: Tensor) -> Tensor:
+        b = self._bound
+        if b is not None and b.native is not None and not torch.compiler.is_compiling():
+            y = b.native.run(x, self.__dict__)
+            if y is not None:
+                return y
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.bfloat16:
@@ -110,6 +115,7 @@ class Int8ScaledLinear(nn.Module):
             b = self._bound = ops.BoundLinearW8a8(
                 key=key, held=ts, weight=self.weight, weight_scale=self.weight_scale, bias=self.bias,
                 static=self.input_scale, pertensor=self.gemm_mode == "pertensor", out_dtype=self.compute_dtype)
+            b.native = ops.native_w8a8(self)
         return b(x2)
 
     def _apply(self, fn: Any, recurse: bool = True) -> "Int8ScaledLinear":

@@ -1,0 +1,187 @@
+"""The native host calls (``csrc/host_calls.cpp``) against the Python bodies they stand for: the operators' native CUDA
+kernels and the layers' native calls give the same bits, and whatever does not fit them is decided, and refused, by
+the general path as before."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _lib():
+    from gen_worker_amd import _native
+
+    _native.load()
+    assert torch.cuda.is_available()
+    yield
+
+
+def _same(a, b):
+    return a.dtype == b.dtype and a.shape == b.shape and torch.equal(a.contiguous().view(torch.uint8),
+                                                                      b.contiguous().view(torch.uint8))
+
+
+def _operands(m, n, k, r, seed=0):
+    from gen_worker_amd import synthetic
+
+    layer = synthetic.w4a4_layer(n, k, r, seed_offset=seed)
+    x = synthetic.activation(m, k, outlier_frac=0.01, outlier_scale=20.0, seed=seed).to(DEV)
+    return x, layer
+
+
+@pytest.mark.parametrize("m,n,k,r,smooth,bias", [(1, 16, 64, 16, True, True), (77, 272, 448, 32, False, False),
+                                                 (300, 384, 640, 64, True, False)])
+def test_operator_kernels_equal_the_python_bodies(m, n, k, r, smooth, bias):
+    from gen_worker_amd import ops
+
+    x, layer = _operands(m, n, k, r, seed=m)
+    sm = layer.smooth.to(DEV) if smooth else None
+    one, second = torch.ones((), device=DEV), torch.full((1,), 0.75, device=DEV)
+    cg = torch.ops.cozy_gen_worker
+    q, s = cg.svdq_quant(x, sm, one, False)
+    q0, s0 = ops._svdq_quant_body(x, sm, one, False)
+    assert _same(q, q0) and _same(s, s0)
+    la = (x @ layer.proj_down.to(DEV)).contiguous()
+    args = (q, s, layer.qweight.to(DEV).t().contiguous(), layer.wscales.to(DEV), one, second, la, layer.proj_up.to(DEV),
+            layer.bias.to(DEV) if bias else None)
+    assert _same(cg.svdq_gemm_w4a4_lora(*args), ops._svdq_gemm_w4a4_lora_body(*args))
+    # operands the native kernels leave to the bodies: a bf16 scale, a per-channel second scale in bf16
+    q1, s1 = cg.svdq_quant(x, sm, one.to(torch.bfloat16), False)
+    assert _same(q1, q0) and _same(s1, s0)
+    per = torch.linspace(0.5, 1.5, n, device=DEV).to(torch.bfloat16)
+    args = args[:5] + (per,) + args[6:]
+    assert _same(cg.svdq_gemm_w4a4_lora(*args), ops._svdq_gemm_w4a4_lora_body(*args))
+
+
+def test_operator_refusals_are_the_bodies_own():
+    from gen_worker_amd import ops
+
+    x, layer = _operands(8, 64, 128, 16)
+    one = torch.ones((), device=DEV)
+    cg = torch.ops.cozy_gen_worker
+    with pytest.raises(ops.SvdqOpError, match="blocked"):
+        cg.svdq_quant(x, None, one, True)
+    with pytest.raises(ops.SvdqOpError, match="dtype"):
+        cg.svdq_quant(x.float(), None, one, False)
+    with pytest.raises(ops.SvdqOpError, match="contiguous"):
+        cg.svdq_quant(torch.cat([x, x], dim=1)[:, :128], None, one, False)
+    with pytest.raises(ops.SvdqOpError, match="one value"):
+        cg.svdq_quant(x, None, torch.ones(2, device=DEV), False)
+    q, s = cg.svdq_quant(x, None, one, False)
+    wq, ws = layer.qweight.to(DEV).t().contiguous(), layer.wscales.to(DEV)
+    la, up = torch.zeros(8, 16, device=DEV, dtype=torch.bfloat16), layer.proj_up.to(DEV)
+    with pytest.raises(ops.SvdqOpError):
+        cg.svdq_gemm_w4a4_lora(q, s, wq, ws, one, torch.ones(1, device=DEV), la[:4], up, None)
+    with pytest.raises(ops.SvdqOpError):
+        cg.svdq_gemm_w4a4_lora(q, s.float(), wq, ws, one, torch.ones(1, device=DEV), la, up, None)
+
+
+class _Ops(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def _awq(n, k, bias=True):
+    from gen_worker_amd.awq import AwqPackedLinear
+
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    mod = AwqPackedLinear(k, n, bias=bias, device=DEV)
+    with torch.no_grad():
+        mod.weight.copy_(torch.randint(0, 256, mod.weight.shape, generator=g, device=DEV, dtype=torch.int32))
+        mod.wscales.copy_(torch.rand(mod.wscales.shape, generator=g, device=DEV) * 0.01)
+        mod.wzeros.copy_(torch.randn(mod.wzeros.shape, generator=g, device=DEV) * 0.02)
+        if bias:
+            mod.bias.copy_(torch.randn(n, generator=g, device=DEV))
+    return mod
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_awq_layer_equals_the_operator(bias):
+    from gen_worker_amd import ops
+
+    n, k = 144, 384
+    mod = _awq(n, k, bias)
+    op = lambda x: torch.ops.cozy_gen_worker.awq_w4a16_mm(  # noqa: E731
+        x.reshape(-1, k).contiguous(), mod.weight, mod.wscales, mod.wzeros, mod.bias)
+    for m in (0, 1, 5, ops.AWQ_GEMV_MAX_M, ops.AWQ_GEMV_MAX_M + 1):
+        x = torch.randn(m, k, device=DEV).to(torch.bfloat16)
+        assert _same(mod(x), op(x)), m
+    x3 = torch.randn(2, 3, k, device=DEV).to(torch.bfloat16)
+    y = mod(x3)
+    assert tuple(y.shape) == (2, 3, n) and _same(y.reshape(6, n), op(x3))
+    wide = torch.randn(3, 2 * k, device=DEV).to(torch.bfloat16)[:, :k]
+    assert _same(mod(wide), op(wide))
+    y0 = mod(x3)
+    with torch.no_grad():
+        mod.weight.data = mod.weight.data.clone() ^ 1   # new storage: read anew by every call
+    assert not torch.equal(mod(x3), y0) and _same(mod(x3).reshape(6, n), op(x3))
+    mode = _Ops()
+    with mode:
+        mod(x3)
+    assert any("awq_w4a16_mm" in o for o in mode.seen), mode.seen
+    with torch.inference_mode():
+        assert _same(mod(x3).reshape(6, n), op(x3))
+    with pytest.raises(Exception, match="dtype"):
+        mod(x3.float())
+
+
+@pytest.mark.parametrize("kind", ["w4a4", "w8a8"])
+def test_layers_native_call_follows_the_module(kind):
+    """After the first forward the native call runs; an operand of another shape or device under the same attribute,
+    a LoRA addend, an in-place weight update and a mode all leave it for the general path."""
+    from gen_worker_amd import synthetic
+    from gen_worker_amd.svdq import build_svdq_w4a4_linear
+    from gen_worker_amd.w8a8 import build_int8_linear
+
+    n, k = 272, 448
+    x, layer = _operands(40, n, k, 32)
+    if kind == "w4a4":
+        mod = build_svdq_w4a4_linear(qweight=layer.qweight, wscales=layer.wscales, smooth=layer.smooth,
+                                     proj_down=layer.proj_down, proj_up=layer.proj_up, bias=layer.bias, device=DEV)
+        name = "svdq_forward_fp6"
+    else:
+        w8 = synthetic.w8a8_layer(n, k)
+        mod = build_int8_linear(qweight=w8.qweight, weight_scale=w8.weight_scale, bias=w8.bias, device=DEV)
+        name = "w8a8_scaled_mm"
+    ref = mod(x)
+    native = mod._bound.native
+    got = native.run(x, mod.__dict__)
+    assert got is not None and _same(got, ref)
+    got = native.run(x.reshape(2, 20, k), mod.__dict__)
+    assert _same(got, ref.reshape(2, 20, n))
+    xr = x.clone().requires_grad_()
+    with torch.enable_grad():
+        assert native.run(xr, mod.__dict__) is None
+    assert native.run(x.float(), mod.__dict__) is None and native.run(x[:, :64], mod.__dict__) is None
+    assert native.run(x.cpu(), mod.__dict__) is None and native.run(x[:0], mod.__dict__) is None
+    mode = _Ops()
+    with mode:
+        assert native.run(x, mod.__dict__) is None
+        assert _same(mod(x), ref)
+    assert any(name in o for o in mode.seen), mode.seen
+    if kind == "w4a4":
+        with torch.no_grad():
+            mod.weight.copy_(mod.weight.flip(0).clone())
+        assert native.run(x, mod.__dict__) is None   # the fp6 records are another weight's now
+        assert not torch.equal(mod(x), ref)
+    else:
+        mod.lora_a = torch.randn(8, k, device=DEV).to(torch.bfloat16)
+        mod.lora_b = torch.randn(n, 8, device=DEV).to(torch.bfloat16)
+        assert native.run(x, mod.__dict__) is None
+        assert _same(mod(x), ref + mod._lora_addend(x))
+        mod.lora_a = mod.lora_b = None
+        assert _same(mod(x), ref)
+    bias = mod.bias
+    mod.bias = None
+    assert native.run(x, mod.__dict__) is None
+    mod.bias = bias
