@@ -486,7 +486,8 @@ int64_t gwa_nvfp4_blocked_scale_numel(int64_t rows, int64_t kblocks);
  *           entries are written; the caller zeroes the padding)
  *   xdq     bf16 [M, K] (out, or NULL): code * e4m3 scale (exact), the
  *           operand of the lane's bf16 GEMM (torch._scaled_mm's product,
- *           models/w4a4.py:173-180, without s2) */
+ *           models/w4a4.py:173-180, without s2)
+ * With xdq, q and scales may both be NULL (only the values are written). */
 int gwa_nvfp4_quant_act(const void* x, int64_t ldx, const float* s2, uint8_t* q, uint8_t* scales,
                         int scale_layout, void* xdq, int64_t M, int64_t K, void* stream);
 

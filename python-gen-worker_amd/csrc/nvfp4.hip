@@ -23,7 +23,7 @@
 // (exact), the operand of the bf16 GEMM.
 //
 // Two lanes per block: 16 bytes of x in per lane, 4 bytes of codes and 16 of
-// bf16 values out, one scale byte per pair: HBM-bound.
+// bf16 values out, one scale byte per pair.
 #include <algorithm>
 
 #include "gwa_common.h"
@@ -42,14 +42,7 @@ __device__ __forceinline__ float e2m1_value(uint32_t code) {
 
 // fp32 in [2^-9, 448] -> e4m3fn bits (bias 7, 3 mantissa bits), round to nearest, ties to even
 __device__ __forceinline__ uint32_t e4m3_rne(float v) {
-  const uint32_t u = __float_as_uint(v);
-  const int e = (int)(u >> 23) - 127;
-  if (e < -6) return (uint32_t)rintf(v * 512.0f);  // subnormal grid 2^-9 (8 = the smallest normal, code 8)
-  const uint32_t m = u & 0x7FFFFFu;
-  uint32_t r = m >> 20;
-  const uint32_t rem = m & 0xFFFFFu;
-  if (rem > 0x80000u || (rem == 0x80000u && (r & 1u))) ++r;
-  return ((uint32_t)(e + 7) << 3) + r;  // r == 8 carries into the exponent
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false) & 0xFFu;
 }
 
 constexpr uint32_t kE4m3Nan = 0x7Fu;  // e4m3fn has no infinity: S.1111.111 is NaN
@@ -82,17 +75,28 @@ __device__ __forceinline__ int64_t blocked_index(int64_t r, int64_t c, int64_t n
 // initialised accumulator, no atomics); the quantizer's workgroups each fold the partials again.
 constexpr int NV_MAX_PARTS = 1024;
 
+// Bound by latency at the sizes layers have (28 MB in 7.2 us with one load in flight per thread): four loads are, and a
+// row index is formed only for rows with a gap between them (a 64-bit division per load).
 __global__ __launch_bounds__(NV_THREADS) void nvfp4_absmax_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                   int64_t M, int K, float* __restrict__ part) {
   __shared__ uint32_t red[NV_THREADS / 64];
-  const int64_t chunks = M * (K / 8);
+  const int64_t chunks = M * (K / 8), step = (int64_t)gridDim.x * NV_THREADS;
+  const bool gap = ldx != K;
   uint32_t mx = 0u;
-  for (int64_t i = (int64_t)blockIdx.x * NV_THREADS + threadIdx.x; i < chunks; i += (int64_t)gridDim.x * NV_THREADS) {
-    const int64_t row = i / (K / 8);
-    const int col = (int)(i - row * (K / 8)) * 8;
-    const v4i w = *(const v4i*)(x + row * ldx + col);
+  for (int64_t i0 = (int64_t)blockIdx.x * NV_THREADS + threadIdx.x; i0 < chunks; i0 += 4 * step) {
+    v4i w[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) mx = max(mx, max(abs_bits(bf16_lo((uint32_t)w[j])), abs_bits(bf16_hi((uint32_t)w[j]))));
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = min(i0 + u * step, chunks - 1);  // past the end: the last chunk again
+      int64_t off = 8 * i;
+      if (gap) off += (i / (K / 8)) * (ldx - K);
+      w[u] = *(const v4i*)(x + off);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        mx = max(mx, max(abs_bits(bf16_lo((uint32_t)w[u][j])), abs_bits(bf16_hi((uint32_t)w[u][j]))));
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
@@ -121,8 +125,55 @@ __device__ __forceinline__ float nvfp4_dynamic_s2(const float* __restrict__ part
   return s != s ? s : fmaxf(s, 1e-12f);  // the reference's clamp keeps a NaN
 }
 
+// e2m1 codes of v[0..7] / den as eight nibbles; mb: the bits of the block's max |v|. The quotient is the correctly
+// rounded one from a correctly rounded reciprocal and one residual step (the residual of a quotient within two units
+// in the last place is exact in one fma, and the correction's own error is below 2^-23 of such a unit); + 0 makes the
+// quotient of -0 a +0, whose sign bit the reference leaves clear. The hardware's conversion (round to nearest even,
+// saturating at 6) then is the reference's count of bounds and tie bumps but for the ties 2.5 and 3.5, which the
+// reference takes to 3. A wave whose den or mb is no ordinary number takes the reference's own steps.
+__device__ __forceinline__ uint32_t e2m1_codes8(const float (&v)[8], float den, uint32_t mb) {
+  const bool plain = den >= 0x1p-60f && den <= 0x1p16f && mb < 0x7F800000u;
+  uint32_t codes = 0;
+  if (__builtin_expect(__any(!plain), 0)) {
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+      float x = v[0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) x = i == j ? v[j] : x;
+      codes |= e2m1_code(x / den) << (4 * i);
+    }
+    return codes;
+  }
+  const float r = 1.0f / den;
+  float q[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float q0 = fmaf(v[i], r, 0.0f);
+    const float q1 = fmaf(fmaf(-q0, den, v[i]), r, q0);
+    q[i] = fabsf(fabsf(q1) - 3.0f) == 0.5f ? __builtin_copysignf(3.0f, q1) : q1;
+  }
+  codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, q[0], q[1], 1.0f, 0);
+  codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, q[2], q[3], 1.0f, 1);
+  codes = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, q[4], q[5], 1.0f, 2);
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(codes, q[6], q[7], 1.0f, 3);
+}
+
+// two e2m1 codes (byte j of codes) * sa as a bf16 pair (exact)
+template <int j>
+__device__ __forceinline__ uint32_t e2m1_pair_value(uint32_t codes, float sa) {
+  typedef float v2f_ __attribute__((ext_vector_type(2)));
+  const v2f_ d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, j);
+  return (__float_as_uint(d[0] * sa) >> 16) | (__float_as_uint(d[1] * sa) & 0xFFFF0000u);
+}
+
 // Two lanes per block (lane pair 2p, 2p + 1 holds its elements 0-7 and 8-15), so every load and store of a
-// wave covers one contiguous run; the block maximum is one exchange within the pair.
+// wave covers one contiguous run; the block maximum is one exchange within the pair. A workgroup takes NV_HALVES
+// runs of 256 half-blocks, their loads issued before the partial maxima are folded. It was bound by VALU work (an IEEE
+// division and ten compares per element, a 64-bit division per half-block, one run per workgroup): 26.9 us at
+// 4608 x 3072 with codes, scales and values written; values alone 14.0 now (2 x 28 MB: 4.0 TB/s, where a plain copy
+// of the array takes 8.4 us from the cache). q and scales may both be absent (values only).
+constexpr int NV_HALVES = 4;
+
 __global__ __launch_bounds__(NV_THREADS) void nvfp4_quant_act_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                      const float* __restrict__ s2p,
                                                                      uint8_t* __restrict__ q,
@@ -130,50 +181,56 @@ __global__ __launch_bounds__(NV_THREADS) void nvfp4_quant_act_kernel(const uint1
                                                                      uint16_t* __restrict__ xdq, int64_t M, int KB,
                                                                      const float* __restrict__ parts, int nparts,
                                                                      float* __restrict__ s2_out) {
-  // dynamic s2: every workgroup folds the partial maxima (before any thread leaves)
+  const int64_t total = 2 * M * KB;  // half-blocks; even, so a pair is active together
+  const int64_t t0 = (int64_t)blockIdx.x * (NV_THREADS * NV_HALVES) + threadIdx.x;
+  const bool rows = ldx != 16 * (int64_t)KB;  // rows with a gap between them
+  v4i w[NV_HALVES];
+#pragma unroll
+  for (int u = 0; u < NV_HALVES; ++u) {
+    const int64_t t = min(t0 + u * NV_THREADS, total - 2 + (threadIdx.x & 1));  // past the end: the last pair again
+    int64_t off = 8 * t;
+    if (rows) off += (t >> 1) / KB * (ldx - 16 * (int64_t)KB);
+    w[u] = *(const v4i*)(x + off);
+  }
+  // dynamic s2: every workgroup folds the partial maxima
   const float s2 = parts ? nvfp4_dynamic_s2(parts, nparts) : *s2p;
   if (parts && blockIdx.x == 0 && threadIdx.x == 0) *s2_out = s2;
-  const int64_t t = (int64_t)blockIdx.x * NV_THREADS + threadIdx.x;  // half-block index over [M, KB, 2]
-  if (t >= 2 * M * KB) return;  // the total is even: a pair is active together
-  const int64_t b = t >> 1;
-  const int h = (int)(t & 1);
-  const int64_t row = b / KB;
-  const int c = (int)(b - row * KB);
-  const v4i w = *(const v4i*)(x + row * ldx + 16 * c + 8 * h);
-  float v[8];
+  const float s2x6 = 6.0f * s2;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[2 * j] = bf16_lo((uint32_t)w[j]);
-    v[2 * j + 1] = bf16_hi((uint32_t)w[j]);
-  }
-  uint32_t mb = 0u;
+  for (int u = 0; u < NV_HALVES; ++u) {
+    const int64_t t = t0 + u * NV_THREADS, b = t >> 1;
+    const int h = (int)(t & 1);
+    float v[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) mb = max(mb, abs_bits(v[i]));
-  mb = max(mb, (uint32_t)__shfl_xor((int)mb, 1));
-  const float tq = __uint_as_float(mb) / (6.0f * s2);
-  // a NaN block maximum (or s2) stays NaN through the reference's clamp and casts to the NaN code
-  const uint32_t sc = tq != tq ? kE4m3Nan : e4m3_rne(fminf(fmaxf(tq, 1.0f / 512.0f), 448.0f));
-  const float sa = e4m3_value(sc);
-  const float den = sa * s2;
-  uint32_t codes = 0;
-  uint32_t dq[4];
+    for (int j = 0; j < 4; ++j) {
+      v[2 * j] = bf16_lo((uint32_t)w[u][j]);
+      v[2 * j + 1] = bf16_hi((uint32_t)w[u][j]);
+    }
+    uint32_t mb = 0u;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t code = e2m1_code(v[i] / den);
-    codes |= code << (4 * i);
+    for (int i = 0; i < 8; ++i) mb = max(mb, abs_bits(v[i]));
+    mb = max(mb, (uint32_t)__shfl_xor((int)mb, 1));
+    const float tq = __uint_as_float(mb) / s2x6;
+    // a NaN block maximum (or s2) stays NaN through the reference's clamp and casts to the NaN code
+    const uint32_t sc = tq != tq ? kE4m3Nan : e4m3_rne(fminf(fmaxf(tq, 1.0f / 512.0f), 448.0f));
+    const float sa = e4m3_value(sc);
+    const uint32_t codes = e2m1_codes8(v, sa * s2, mb);
+    if (t >= total) break;
+    if (q) *(uint32_t*)(q + b * 8 + 4 * h) = codes;
+    if (scales && h == 0) {
+      int64_t at = b;
+      if (blocked) {
+        const int64_t row = b / KB;
+        at = blocked_index(row, b - row * KB, (KB + 3) / 4);
+      }
+      scales[at] = (uint8_t)sc;
+    }
     if (xdq) {
-      const float d = e2m1_value(code) * sa;  // exact in bf16
-      const uint32_t bits = __float_as_uint(d) >> 16;
-      if (i & 1) dq[i >> 1] |= bits << 16;
-      else dq[i >> 1] = bits;
+      const uint32_t dq[4] = {e2m1_pair_value<0>(codes, sa), e2m1_pair_value<1>(codes, sa),
+                              e2m1_pair_value<2>(codes, sa), e2m1_pair_value<3>(codes, sa)};
+      *(v4i*)(xdq + b * 16 + 8 * h) = (v4i){(int)dq[0], (int)dq[1], (int)dq[2], (int)dq[3]};
     }
   }
-  *(uint32_t*)(q + b * 8 + 4 * h) = codes;
-  if (h == 0) {
-    const int64_t ncb = (KB + 3) / 4;
-    scales[blocked ? blocked_index(row, c, ncb) : b] = (uint8_t)sc;
-  }
-  if (xdq) *(v4i*)(xdq + b * 16 + 8 * h) = (v4i){(int)dq[0], (int)dq[1], (int)dq[2], (int)dq[3]};
 }
 
 // codes [rows, K/2] + e4m3 scales (flat or blocked) -> bf16 [rows, K] = code * scale (exact)
@@ -203,29 +260,37 @@ __global__ __launch_bounds__(NV_THREADS) void nvfp4_dequant_kernel(const uint8_t
 
 // y (bf16 [M, N], in place) = RN_bf16(RN_bf16(y * c) + bias), c = RN_bf16(s2 * ws2): the module's
 // `y * (s2 * weight_scale_2).to(y.dtype)` then `+ bias` (models/w4a4.py:349-351), each rounded to bf16 as
-// torch's bf16 ops round; 8 elements per thread
+// torch's bf16 ops round. A workgroup is tx (columns of 8) x ty threads (a power of two each) and takes SB_ROWS rows
+// of every thread's column: the bias is loaded once for them, their loads are in flight together, and no column is
+// found by a 64-bit remainder (12.1 us at 4608 x 3072 with one column of one row per thread, 10.5 so).
+constexpr int SB_ROWS = 4;
+
 __global__ __launch_bounds__(NV_THREADS) void nvfp4_scale_bias_kernel(uint16_t* __restrict__ y,
                                                                       const float* __restrict__ s2,
                                                                       const float* __restrict__ ws2,
                                                                       const uint16_t* __restrict__ bias, int64_t M,
                                                                       int N) {
-  const int64_t i = ((int64_t)blockIdx.x * NV_THREADS + threadIdx.x) * 8;
-  if (i >= M * N) return;
-  const float c = bf16_to_f32(f32_to_bf16(*s2 * *ws2));
-  const int n0 = (int)(i % N);
-  v4i w = *(const v4i*)(y + i);
-  v4i b = bias ? *(const v4i*)(bias + n0) : (v4i){0, 0, 0, 0};
+  const int n = 8 * (int)(blockIdx.y * blockDim.x + threadIdx.x);
+  const int64_t r0 = ((int64_t)blockIdx.x * SB_ROWS) * blockDim.y + threadIdx.y;
+  if (n >= N || r0 >= M) return;
+  v4i w[SB_ROWS];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float lo = bf16_to_f32(f32_to_bf16(bf16_lo((uint32_t)w[j]) * c));
-    float hi = bf16_to_f32(f32_to_bf16(bf16_hi((uint32_t)w[j]) * c));
-    if (bias) {
-      lo += bf16_lo((uint32_t)b[j]);
-      hi += bf16_hi((uint32_t)b[j]);
+  for (int u = 0; u < SB_ROWS; ++u)  // rows past the last: the last again
+    w[u] = *(const v4i*)(y + min(r0 + u * (int64_t)blockDim.y, M - 1) * N + n);
+  const v4i b = bias ? *(const v4i*)(bias + n) : (v4i){0, 0, 0, 0};
+  const float c = bf16_to_f32(f32_to_bf16(*s2 * *ws2));
+#pragma unroll
+  for (int u = 0; u < SB_ROWS; ++u) {
+    const int64_t r = r0 + u * (int64_t)blockDim.y;
+    if (r >= M) break;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t p = pack_bf16x2_rn(bf16_lo((uint32_t)w[u][j]) * c, bf16_hi((uint32_t)w[u][j]) * c);
+      if (bias) p = pack_bf16x2_rn(bf16_lo(p) + bf16_lo((uint32_t)b[j]), bf16_hi(p) + bf16_hi((uint32_t)b[j]));
+      w[u][j] = (int)p;
     }
-    w[j] = (int)pack_bf16x2_rn(lo, hi);
+    *(v4i*)(y + r * N + n) = w[u];
   }
-  *(v4i*)(y + i) = w;
 }
 
 }  // namespace
@@ -239,10 +304,14 @@ extern "C" int gwa_nvfp4_scale_bias(void* y, const float* s2, const float* ws2, 
   GWA_REQUIRE(y && s2 && ws2, "%s: null pointer", what);
   GWA_REQUIRE(GWA_ALIGNED(y, 16) && GWA_ALIGNED(bias, 16) && GWA_ALIGNED(s2, 4) && GWA_ALIGNED(ws2, 4),
               "%s: y and bias must be 16-byte aligned", what);
-  const int64_t threads = M * N / 8;
-  hipLaunchKernelGGL(nvfp4_scale_bias_kernel, dim3((unsigned)((threads + NV_THREADS - 1) / NV_THREADS)),
-                     dim3(NV_THREADS), 0, (hipStream_t)stream, (uint16_t*)y, s2, ws2, (const uint16_t*)bias, M,
-                     (int)N);
+  int tx = 16;
+  while (tx < NV_THREADS && tx < N / 8) tx *= 2;
+  const int ty = NV_THREADS / tx;
+  const int64_t gx = (M + SB_ROWS * ty - 1) / (SB_ROWS * ty), gy = (N / 8 + tx - 1) / tx;
+  GWA_REQUIRE(gx < (1ll << 31) && gy < 65536 && N < (1ll << 31), "%s: [%lld, %lld] is too large", what, (long long)M,
+              (long long)N);
+  hipLaunchKernelGGL(nvfp4_scale_bias_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(tx, ty), 0, (hipStream_t)stream,
+                     (uint16_t*)y, s2, ws2, (const uint16_t*)bias, M, (int)N);
   return gwa_check_launch(what);
 }
 
@@ -261,7 +330,7 @@ static int nvfp4_quant(const char* what, const void* x, int64_t ldx, const float
               "%s: scale_layout %d", what, scale_layout);
   GWA_REQUIRE(M * K < (1ll << 40), "%s: shape too large", what);
   if (M == 0) return GWA_OK;
-  GWA_REQUIRE(x && (s2 || (s2_out && parts)) && q && scales, "%s: null pointer", what);
+  GWA_REQUIRE(x && (s2 || (s2_out && parts)) && ((q && scales) || (!q && !scales && xdq)), "%s: null pointer", what);
   GWA_REQUIRE(GWA_ALIGNED(x, 16) && GWA_ALIGNED(q, 8) && GWA_ALIGNED(s2, 4) && GWA_ALIGNED(s2_out, 4) &&
                   GWA_ALIGNED(parts, 4) && GWA_ALIGNED(xdq, 16),
               "%s: x and xdq must be 16-byte, q 8-byte aligned", what);
@@ -276,7 +345,7 @@ static int nvfp4_quant(const char* what, const void* x, int64_t ldx, const float
     if (rc != GWA_OK) return rc;
   }
   const int64_t halves = 2 * M * (K / 16);
-  hipLaunchKernelGGL(nvfp4_quant_act_kernel, dim3((unsigned)((halves + NV_THREADS - 1) / NV_THREADS)),
+  hipLaunchKernelGGL(nvfp4_quant_act_kernel, dim3((unsigned)((halves + NV_THREADS * NV_HALVES - 1) / (NV_THREADS * NV_HALVES))),
                      dim3(NV_THREADS), 0, st, (const uint16_t*)x, ldx, s2, q, scales,
                      scale_layout == GWA_NVFP4_SCALES_BLOCKED ? 1 : 0, (uint16_t*)xdq, M, (int)(K / 16), parts,
                      nparts, s2_out);

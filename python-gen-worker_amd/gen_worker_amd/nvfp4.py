@@ -142,9 +142,9 @@ class Nvfp4Linear(nn.Module):
             x2 = x2 * self.pre_quant_scale
         if self.input_scale is not None:
             s2 = self.input_scale.reshape(())
-            _, _, xdq = torch.ops.cozy_gen_worker.nvfp4_quant_act(x2.contiguous(), s2, False, True)
+            xdq, _ = torch.ops.cozy_gen_worker.nvfp4_act_values(x2.contiguous(), s2)
         else:   # s2 = max|x| / (6 * 448) computed on the device, in the quantizer's launch
-            _, _, xdq, s2 = torch.ops.cozy_gen_worker.nvfp4_quant_act_dyn(x2.contiguous(), False, True)
+            xdq, s2 = torch.ops.cozy_gen_worker.nvfp4_act_values(x2.contiguous(), None)
         y = F.linear(xdq, self.weight_dq)
         torch.ops.cozy_gen_worker.nvfp4_scale_bias(y, s2, self.weight_scale_2.reshape(()), self.bias)
         return y.reshape(*shape[:-1], self.out_features)

@@ -1369,6 +1369,42 @@ def _(x2, blocked, dequant):
             x2.new_empty((), dtype=torch.float32))
 
 
+@torch.library.custom_op("cozy_gen_worker::nvfp4_act_values", mutates_args=())
+def nvfp4_act_values(x2: Tensor, s2: Optional[Tensor]) -> tuple[Tensor, Tensor]:
+    """The dequantized bf16 activations of ``nvfp4_quant_act`` (``s2`` given) or ``nvfp4_quant_act_dyn`` (None)
+    alone, without writing the codes and scales a layer's product does not read, and the dynamic s2 (an empty
+    tensor where ``s2`` is given)."""
+    name = "nvfp4_act_values"
+    if x2.dim() != 2:
+        raise SvdqOpError(f"{name}: x2 must be 2-D, got {tuple(x2.shape)}")
+    _check_dtype(name, x2, torch.bfloat16, what="x2")
+    s2 = _scalar_f32(name, s2)
+    if x2.stride(1) != 1 or x2.stride(0) % 8:
+        x2 = x2.contiguous()
+    _check_cuda(name, s2=s2)
+    if not x2.is_cuda:
+        raise SvdqOpError(f"{name}: x2 is on {x2.device}; the nvfp4 lane runs on the GPU only")
+    m, k = int(x2.shape[0]), int(x2.shape[1])
+    if k % NVFP4_BLOCK:
+        raise SvdqOpError(f"{name}: K={k} is not a multiple of {NVFP4_BLOCK}")
+    xdq = torch.empty(m, k, dtype=torch.bfloat16, device=x2.device)
+    if s2 is not None:
+        nat.call("gwa_nvfp4_quant_act", nat.ptr(x2), int(x2.stride(0)), nat.ptr(s2), None, None, nat.NVFP4_SCALES_FLAT,
+                 nat.ptr(xdq), m, k, nat.stream_of(x2))
+        return xdq, torch.empty(0, dtype=torch.float32, device=x2.device)
+    s2o = torch.empty((), dtype=torch.float32, device=x2.device)
+    parts = torch.empty(NVFP4_MAX_PARTS, dtype=torch.float32, device=x2.device)
+    nat.call("gwa_nvfp4_quant_act_dyn", nat.ptr(x2), int(x2.stride(0)), nat.ptr(s2o), nat.ptr(parts), None, None,
+             nat.NVFP4_SCALES_FLAT, nat.ptr(xdq), m, k, nat.stream_of(x2))
+    return xdq, s2o
+
+
+@nvfp4_act_values.register_fake
+def _(x2, s2):
+    s2o = x2.new_empty((), dtype=torch.float32) if s2 is None else x2.new_empty(0, dtype=torch.float32)
+    return x2.new_empty(int(x2.shape[0]), int(x2.shape[1])), s2o
+
+
 @torch.library.custom_op("cozy_gen_worker::quant_nvfp4_act", mutates_args=())
 def quant_nvfp4_act(x2: Tensor, s2: Tensor) -> tuple[Tensor, Tensor]:
     """The reference op's contract (models/nvfp4_quant.py:185-187): (packed codes [M, K/2], e4m3 scales in the

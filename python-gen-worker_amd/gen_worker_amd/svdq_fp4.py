@@ -173,7 +173,7 @@ class SvdqFp4Linear(nn.Module):
         x2 = x.reshape(-1, self.in_features).contiguous()
         xs = x2 if self.smooth_factor is None else x2 / self.smooth_factor
         # codes, micro-scales and the exact values code * scale, with s2 = max|xs| / (6 * 448) on the device
-        _, _, xdq, s2 = torch.ops.cozy_gen_worker.nvfp4_quant_act_dyn(xs.contiguous(), False, True)
+        xdq, s2 = torch.ops.cozy_gen_worker.nvfp4_act_values(xs.contiguous(), None)
         y = F.linear(xdq, self.weight_dq)
         y = y * (s2 * self.weight_scale_2).to(y.dtype)
         if self.proj_down is not None:

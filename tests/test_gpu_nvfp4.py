@@ -188,3 +188,56 @@ def test_scale_bias_bit_exact(bias):
     if bias:
         want = N.bf16_round(want + b)
     assert np.array_equal(yd.float().cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+def _near_rows(k, s2v):
+    """Rows of one scale (block maximum 6 * s2: scale 1, so q = x / s2) whose other values lie on, just below and just
+    above every bound of the code grid, as close as bf16 comes for this s2, both signs and zeros."""
+    rows = []
+    for bound in (0.25, 0.5, 0.75, 1.0, 1.25, 1.75, 2.5, 3.5, 5.0):
+        c = N.bf16_round(np.float32(bound * s2v))
+        u = np.array([c], np.float32).view(np.uint32)[0] >> 16
+        near = ((np.arange(-3, 4) + int(u)).astype(np.uint32) << 16).view(np.float32)
+        blk = np.concatenate([[6.0 * s2v], near, -near, [-0.0]]).astype(np.float32)[:16]
+        rows.append(np.tile(blk, k // 16))
+    return N.bf16_round(np.stack(rows))
+
+
+@pytest.mark.parametrize("s2v", [1.0, 0.75, 0.0123, 1.0 / 3.0, 2.0 ** -20, 1e-12, 1e6, 1 + 2.0 ** -23, 1 - 2.0 ** -24,
+                                 1 - 2.0 ** -23, 1.5 + 2.0 ** -23, 1.5 - 2.0 ** -23, 1.5 - 2.0 ** -22])
+def test_codes_around_every_bound(s2v):
+    """Values on and either side of each bound, for second scales that make the quotients exact and inexact, lie within a
+    few units of 1 and 1.5 (where a residual step is closest to rounding wrongly), and pass the range it serves."""
+    s2v = np.float32(s2v)
+    x = _near_rows(64, s2v)
+    q, sc, xdq = torch.ops.cozy_gen_worker.nvfp4_quant_act(_bf16(x), torch.tensor(s2v, device=DEV), False, True)
+    oq, osc = N.quantize_activation(x, s2v)
+    assert np.array_equal(sc.cpu().numpy(), osc) and np.array_equal(q.cpu().numpy(), oq)
+    assert np.array_equal(xdq.float().cpu().numpy().view(np.uint32), N.dequantize(oq, osc).view(np.uint32))
+
+
+@pytest.mark.parametrize("m,k", [(1, 16), (5, 4080), (257, 272), (64, 8192)])
+def test_values_alone_equal_the_quantizers(m, k):
+    """nvfp4_act_values against the quantizing ops over ends of a workgroup's runs, contiguous and row-strided."""
+    cg = torch.ops.cozy_gen_worker
+    x = _bf16(_act(m, k, seed=m))
+    wide = torch.cat([x, x[:, :8]], dim=1)[:, :k]
+    s2 = torch.tensor(0.0041, device=DEV)
+    want = cg.nvfp4_quant_act(x, s2, False, True)[2]
+    _, _, dyn, s2d = cg.nvfp4_quant_act_dyn(x, False, True)
+    for a in (x, wide):
+        assert torch.equal(cg.nvfp4_act_values(a, s2)[0], want)
+        v, s = cg.nvfp4_act_values(a, None)
+        assert torch.equal(v, dyn) and torch.equal(s, s2d)
+
+
+@pytest.mark.parametrize("m,n", [(1, 8), (3, 136), (65, 2056), (130, 4096)])
+def test_scale_bias_tile_ends(m, n):
+    g = np.random.default_rng(m + n)
+    y = N.bf16_round((g.standard_normal((m, n)) * 3).astype(np.float32))
+    b = N.bf16_round((g.standard_normal(n) * 0.5).astype(np.float32))
+    s2, ws2 = np.float32(0.0123), np.float32(0.0071)
+    yd = _bf16(y)
+    torch.ops.cozy_gen_worker.nvfp4_scale_bias(yd, torch.tensor(s2, device=DEV), torch.tensor(ws2, device=DEV), _bf16(b))
+    want = N.bf16_round(N.bf16_round(y * N.bf16_round(s2 * ws2)) + b)
+    assert np.array_equal(yd.float().cpu().numpy().view(np.uint32), want.view(np.uint32))
