@@ -185,3 +185,31 @@ def test_layers_native_call_follows_the_module(kind):
     mod.bias = None
     assert native.run(x, mod.__dict__) is None
     mod.bias = bias
+
+
+@pytest.mark.parametrize("m,k", [(1, 64), (3, 448), (4, 512), (5, 576), (130, 1600)])
+@pytest.mark.parametrize("smooth", [None, "normal", "subnormal"])
+def test_quantizer_without_a_low_rank_product_equals_the_oracle(m, k, smooth):
+    """Ends of a wave's four rows and 512 columns; a factor whose reciprocal is not normal takes the division."""
+    import numpy as np
+
+    from gen_worker_amd import synthetic
+    from oracle import svdq_oracle as O
+
+    bits = lambda t: t.contiguous().view(torch.int16).numpy().view(np.uint16)  # noqa: E731
+    x = synthetic.activation(m, k, outlier_frac=0.01, outlier_scale=20.0, seed=m + k)
+    sm = None if smooth is None else synthetic.smooth_factor(k, seed=k)
+    if smooth == "subnormal":
+        sm[k // 2] = 2.0 ** 127
+    wide = torch.cat([x, x[:, :8]], dim=1).to(DEV)[:, :k]
+    one = torch.ones((), device=DEV)
+    want_q, want_s = O.quantize_act_int4(bits(x), None if sm is None else bits(sm))
+    from gen_worker_amd import _native as nat
+
+    for a in (x.to(DEV), wide):
+        q = torch.empty(m, k // 2, dtype=torch.uint8, device=DEV)
+        s = torch.empty(m, k // 64, dtype=torch.float16, device=DEV)
+        smd = None if sm is None else sm.to(DEV)
+        nat.call("gwa_svdq_quant_int4", a.data_ptr(), a.stride(0), nat.ptr(smd), one.data_ptr(), None, 0, nat.QFMT_INT4,
+                 q.data_ptr(), s.data_ptr(), None, m, k, nat.stream_of(a))
+        assert np.array_equal(q.cpu().numpy(), want_q) and np.array_equal(bits(s.cpu()), want_s.view(np.uint16))
