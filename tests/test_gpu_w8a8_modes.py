@@ -98,3 +98,30 @@ def test_module_modes(mode, static):
                         pertensor=mode == "pertensor", static=static)
     check_output(y.reshape(-1, 512), ref, what=f"module {mode} static={static}")
 
+
+
+@pytest.mark.parametrize("m,k", [(1, 64), (5, 3072), (3, 3080), (6, 6144), (2, 6152), (4, 12288), (3, 12296)])
+@pytest.mark.parametrize("pertensor,static", [(False, None), (True, None), (False, 0.037)])
+def test_quantizer_at_the_ends_of_its_register_sizes(m, k, pertensor, static):
+    """Rows on either side of each register size (and the two-pass kernel past them), with a row of zeros, an infinite
+    row and a NaN: the codes and scales of the IEEE division, bit for bit."""
+    g = np.random.default_rng(m * 7 + k)
+    x = (g.standard_normal((m, k)) * np.exp(g.uniform(-6, 3, (m, 1)))).astype(np.float32)
+    x[:, g.integers(0, k, 2)] *= 30.0
+    xb = O.f32_to_bf16_bits(x)
+    xf = O.bf16_bits_to_f32(xb)
+    rows = [xf]
+    if m > 2:
+        z = xf.copy()
+        z[1] = 0.0
+        if not pertensor:
+            z[2, 3] = np.inf
+        rows.append(z)
+    for xr in rows:
+        xd = torch.from_numpy(xr).to(torch.bfloat16).to(DEV)
+        st = None if static is None else torch.tensor([[static]], dtype=torch.float32, device=DEV)
+        q, s = torch.ops.cozy_gen_worker.w8a8_quant(xd, pertensor, st)
+        wq, ws = O.quantize_act_int8(O.f32_to_bf16_bits(xr), pertensor, static)
+        assert np.array_equal(s.cpu().numpy(), ws.reshape(s.shape))
+        fin = np.isfinite(xr).all(axis=1)   # a finite value over an infinite scale is a code 0; inf / inf is not a code
+        assert np.array_equal(q.cpu().numpy()[fin], wq[fin])
