@@ -15,7 +15,9 @@
 // fp32, rounded to bf16.
 //
 // The layer is bound by the weight read (N * K / 2 bytes + the two scale
-// grids); every weight byte is read once per MT activation rows:
+// grids) and by dequantizing it. The GEMV (up to 4 activation rows) reads every
+// weight byte once per MT activation rows; the MFMA kernel (more) once per 16.
+// GEMV:
 //  * a workgroup stages MT activation rows in LDS (bf16) and owns 16 output
 //    rows, one per 16-lane team; lane t of a team takes the 32 codes
 //    [512 s + 32 t, +32) of span s (16 weight bytes, one coalesced 256-byte
@@ -39,6 +41,7 @@ namespace {
 constexpr int AWQ_THREADS = 256, AWQ_TEAMS = AWQ_THREADS / 16;  // 16 output rows per workgroup
 constexpr int AWQ_SPAN = 512;                                    // codes of a row per team step (16 lanes x 32)
 constexpr int AWQ_BATCH = 4;                                     // spans per load batch
+constexpr int AWQ_MFMA_SPAN = 128;                                // codes of a row per wave step of the MFMA kernel
 constexpr int AWQ_LDS_MAX = 64 * 1024;                           // activation rows staged in LDS
 
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
@@ -150,6 +153,62 @@ __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
   }
 }
 
+// More than 4 activation rows: one read of the weight for up to 16 of them, on 16x16x32 MFMA (weights the first operand,
+// activation rows the second: a lane holds 8 consecutive inputs of one row). The GEMV above reads and dequantizes the
+// weight once per 4 rows and spends 4 dot products per 8 codes on each row; here dequantizing (the arithmetic that
+// bounds it at few rows) is done once and the products are one instruction per 8 codes of a lane. A workgroup owns 16
+// output rows, its W waves take every W-th span of 128 inputs, and their sums meet in LDS; activations come straight
+// from memory (staged in LDS they would cost a barrier before the first product and the occupancy that hides the
+// loads: 8 waves per SIMD, no load batches, is the fastest; batches of 2, 3 and 6 spans in flight took 16-18 us at 3072 ->
+// 9216 and 5 rows, 32 and 64 output rows per workgroup 12.9 and 14.1, this 11.5).
+// us, GEMV -> this: 3072 -> 18432 5 rows 25.4 -> 17.9, 16 rows 45 -> 25; 3072 -> 3072 16 rows 11.6 -> 6.4; 12288 ->
+// 3072 16 rows 47.6 -> 20.6.
+template <int W>
+__global__ __launch_bounds__(64 * W) void awq_w4a16_mfma_kernel(
+    const uint16_t* __restrict__ x, int64_t ldx, const uint8_t* __restrict__ weight,
+    const uint16_t* __restrict__ wscales, const uint16_t* __restrict__ wzeros, const uint16_t* __restrict__ bias,
+    uint16_t* __restrict__ out, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) float part[W][256];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16, ng = K >> 6;
+  const rsrc_t xbuf = make_rsrc(x, (uint32_t)(((int64_t)(M - 1) * ldx + K) * 2));
+  const rsrc_t wbuf = make_rsrc(weight, (uint32_t)((int64_t)N * (K >> 1)));
+  const rsrc_t sbuf = make_rsrc(wscales, (uint32_t)((int64_t)N * ng * 2));
+  const rsrc_t zbuf = make_rsrc(wzeros, (uint32_t)((int64_t)N * ng * 2));
+  const uint32_t xoff = (uint32_t)(((int64_t)(m0 + l16) * ldx + 32 * g) * 2);
+  const uint32_t woff = (uint32_t)((int64_t)(n0 + l16) * (K >> 1) + 16 * g);
+  const uint32_t soff = (uint32_t)(((int64_t)(n0 + l16) * ng + (g >> 1)) * 2);
+
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = wave; s < K / AWQ_MFMA_SPAN; s += W) {
+    const float sv = bf16_to_f32(buf_load2(sbuf, soff + 4u * (uint32_t)s));
+    const float zv = bf16_to_f32(buf_load2(zbuf, soff + 4u * (uint32_t)s));
+    const v4i wd = buf_load16(wbuf, woff + (uint32_t)(AWQ_MFMA_SPAN / 2) * (uint32_t)s);
+    v4i xv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      xv[q] = buf_load16(xbuf, m0 + l16 < M ? xoff + (uint32_t)(2 * AWQ_MFMA_SPAN) * (uint32_t)s + 16u * q : kOOB);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t w[4];
+      dequant8((uint32_t)wd[q], sv, zv, w);
+      const v4i wv = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, wv), __builtin_bit_cast(v8bf, xv[q]), acc,
+                                                    0, 0, 0);
+    }
+  }
+  // the block (row 4 g + i, activation row l16) of this wave at [16 l16 + row]; the waves' sums, bias, bf16
+  *(v4f*)&part[wave][16 * l16 + 4 * g] = acc;
+  __syncthreads();
+  const int m = m0 + (tid >> 4), n = n0 + (tid & 15);
+  if (tid >= 256 || m >= M) return;
+  float v = part[0][tid];
+#pragma unroll
+  for (int w = 1; w < W; ++w) v += part[w][tid];
+  out[(int64_t)m * N + n] = f32_to_bf16(v + (bias ? bf16_to_f32(bias[n]) : 0.0f));
+}
+
 // weight [N, K/2] + scales / zeros [N, K/64] -> bf16 [N, K]: one dword of codes (8 columns) per thread
 __global__ __launch_bounds__(256) void awq_w4a16_dequant_kernel(const uint32_t* __restrict__ weight,
                                                                  const uint16_t* __restrict__ wscales,
@@ -177,6 +236,16 @@ int launch_gemv(const void* x, int64_t ldx, const void* weight, const void* ws, 
   return gwa_check_launch("awq_w4a16_mm");
 }
 
+template <int W>
+int launch_mfma(const void* x, int64_t ldx, const void* weight, const void* ws, const void* wz, const void* bias,
+                void* out, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  const dim3 grid((unsigned)(N / 16), (unsigned)((M + 15) / 16));
+  hipLaunchKernelGGL((awq_w4a16_mfma_kernel<W>), grid, dim3(64 * W), 0, st, (const uint16_t*)x, ldx,
+                     (const uint8_t*)weight, (const uint16_t*)ws, (const uint16_t*)wz, (const uint16_t*)bias,
+                     (uint16_t*)out, (int)M, (int)N, (int)K);
+  return gwa_check_launch("awq_w4a16_mm");
+}
+
 }  // namespace
 
 extern "C" int gwa_awq_w4a16_mm(const void* x, int64_t ldx, const void* weight, const void* wscales,
@@ -198,7 +267,16 @@ extern "C" int gwa_awq_w4a16_mm(const void* x, int64_t ldx, const void* weight, 
                   GWA_ALIGNED(bias, 2) && GWA_ALIGNED(out, 2),
               "%s: x must be 16-byte and weight 4-byte aligned", what);
   hipStream_t st = (hipStream_t)stream;
-  // activation rows per workgroup: up to 4, as many as fit the LDS budget
+  // MFMA from 5 rows on (up to 4 the GEMV reads the weight once too, in whole 256-byte row segments: 5 rows at 3072 ->
+  // 18432 25.4 -> 17.9 us, 4 rows 16.4 -> 17.9), except long rows on few output rows: there the GEMV's chunks of rows
+  // are the parallelism (15360 -> 512, 16 rows: GEMV 19.5, MFMA 24.6; 15360 -> 1024 26.6 and 24.9; 8192 -> 512 16.3
+  // and 13.9). 8 waves per workgroup for rows past 4096 inputs (15360 -> 2048, 16 rows: 4 waves 32.4, 8 25.0),
+  // 4 otherwise (3072 -> 18432, 5 rows: 17.9 and 19.5).
+  if (M > 4 && (N >= 1024 || K <= 8192)) {
+    if (K > 4096) return launch_mfma<8>(x, ldx, weight, wscales, wzeros, bias, out, M, N, K, st);
+    return launch_mfma<4>(x, ldx, weight, wscales, wzeros, bias, out, M, N, K, st);
+  }
+  // GEMV, activation rows per workgroup: up to 4, as many as fit the LDS budget
   int mt = M == 1 ? 1 : (M == 2 ? 2 : 4);
   while (mt > 1 && (int64_t)mt * K * 2 > AWQ_LDS_MAX) mt /= 2;
   if (mt == 1) return launch_gemv<1>(x, ldx, weight, wscales, wzeros, bias, out, M, N, K, st);

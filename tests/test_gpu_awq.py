@@ -53,6 +53,24 @@ def test_mm_matches_oracle(m, n, k, bias):
     check_output(y, ref, what=f"awq m={m} n={n} k={k} ({'gemv' if m <= AWQ_GEMV_MAX_M else 'dequant + gemm'})")
 
 
+@pytest.mark.parametrize("m,n,k", [(5, 16, 128), (6, 48, 384), (8, 1008, 8192), (15, 1024, 4096), (16, 1024, 4224),
+                                   (16, 32, 640), (9, 512, 8320), (16, 1008, 15360), (7, 1040, 15360)])
+def test_mm_several_rows(m, n, k):
+    """From five rows on: the MFMA kernel with 4 (k up to 4096) and 8 waves, waves without a span, and the GEMV that
+    keeps long rows on few outputs; a strided x, and each row equal to the same row beside other rows. The products
+    are exact in fp32 and both sides sum K of them, so the bound is that of the GEMV's own test."""
+    codes, s, z, b, t = _layer(n, k, seed=m + n + k)
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    op = torch.ops.cozy_gen_worker.awq_w4a16_mm
+    xd = x.to(DEV)
+    y = op(xd, t["weight"], t["wscales"], t["wzeros"], t["bias"])
+    check_output(y, A.awq_linear(bits16(x), codes, s, z, b), what=f"awq m={m} n={n} k={k}")
+    other = torch.randn(16, k, generator=g).to(torch.bfloat16).to(DEV)
+    other[3] = xd[0]
+    assert torch.equal(op(other, t["weight"], t["wscales"], t["wzeros"], t["bias"])[3], y[0])
+
+
 def test_mm_deterministic_and_row_independent():
     """Repeated calls agree bit for bit, and a row's result does not depend on the other rows of its chunk."""
     _, _, _, _, t = _layer(1024, 3072, seed=3)
