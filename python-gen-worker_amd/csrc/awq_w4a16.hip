@@ -27,10 +27,11 @@
 //    meets the matching activation pair in one v_dot2c_f32_bf16 per
 //    activation row (fp32 accumulation), the activations read as 16 bytes
 //    per lane from LDS, swizzled so the 16 lanes of a team hit distinct banks;
-//  * the first batch of 4 spans is requested before the activations are
-//    staged, later batches as the previous one is consumed; the team's 16
-//    partial sums are reduced by lane exchanges, and lane 0 adds the bias and
-//    stores the bf16 result.
+//  * the activations are requested before the weights, so that staging them
+//    waits for them alone, and every span of a row of up to 4096 inputs is
+//    requested at once (longer rows: batches of 4 spans, two in flight); the
+//    team's 16 partial sums are reduced by lane exchanges, and lane 0 adds the
+//    bias and stores the bf16 result.
 // A second kernel dequantizes the whole weight to bf16 [N, K] (the same
 // values) for callers with many activation rows, which then run a library
 // GEMM.
@@ -40,7 +41,8 @@ namespace {
 
 constexpr int AWQ_THREADS = 256, AWQ_TEAMS = AWQ_THREADS / 16;  // 16 output rows per workgroup
 constexpr int AWQ_SPAN = 512;                                    // codes of a row per team step (16 lanes x 32)
-constexpr int AWQ_BATCH = 4;                                     // spans per load batch
+constexpr int AWQ_BATCH = 4;                                     // spans per load batch of a long row
+constexpr int AWQ_ALL = 8;                                       // rows of up to this many spans load at once
 constexpr int AWQ_MFMA_SPAN = 128;                                // codes of a row per wave step of the MFMA kernel
 constexpr int AWQ_LDS_MAX = 64 * 1024;                           // activation rows staged in LDS
 
@@ -70,7 +72,21 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 // of a lane's 64 bytes (units 4t + i of a span, lanes t = 0..15) then hit 16 distinct bank groups
 __device__ __forceinline__ int x_unit(int u) { return u ^ ((u >> 4) & 3); }
 
-template <int MT>
+// a barrier for the LDS writes alone: loads stay in flight
+__device__ __forceinline__ void barrier_staged() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// B spans per load batch; PIPED: rows of more than B spans, two batches in flight. Loads return in order: with the
+// weights requested first (as this kernel did) no dot product began before the last of them had arrived, and one
+// token at 3072 -> 18432 took the launch and staging (3.9 us), the loads (3.5) and the arithmetic (4.5) one after
+// the other. us, before -> now: 3072 -> 18432, 1 row 11.8 -> 9.7, 2 13.7 -> 11.8, 4 17.8 -> 15.8; 12288 -> 3072, 1 row
+// 14.1 -> 10.4; 15360 -> 18432, 4 rows 117 -> 94. What is left at one row: 3.9 us of launch and staging, 3.5 of loads
+// and 4.5 of arithmetic, now partly over one another.
+template <int MT, int B, bool PIPED>
 __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint8_t* __restrict__ weight,
     const uint16_t* __restrict__ wscales, const uint16_t* __restrict__ wzeros, const uint16_t* __restrict__ bias,
@@ -85,51 +101,65 @@ __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
   const int n = blockIdx.x * AWQ_TEAMS + team;
   const bool row_ok = n < N;
   const int spans = (K + AWQ_SPAN - 1) / AWQ_SPAN, ng = K >> 6;
+  const rsrc_t xbuf = make_rsrc(x, (uint32_t)(((int64_t)(M - 1) * ldx + K) * 2));
   const rsrc_t wbuf = make_rsrc(weight, (uint32_t)((int64_t)N * (K >> 1)));
   const rsrc_t sbuf = make_rsrc(wscales, (uint32_t)((int64_t)N * ng * 2));
   const rsrc_t zbuf = make_rsrc(wzeros, (uint32_t)((int64_t)N * ng * 2));
   const uint32_t wrow = (uint32_t)((int64_t)n * (K >> 1)) + 16u * (uint32_t)t;
   const uint32_t grow = (uint32_t)((int64_t)n * ng + (t >> 1)) * 2u;
 
-  v4i wd[AWQ_BATCH];
-  uint16_t sc[AWQ_BATCH], ze[AWQ_BATCH];
-  auto load_batch = [&](int s0) __attribute__((always_inline)) {
+  // 1. the MT activation rows (rows past M: zeros): the first XU units of each thread into registers, ahead of the
+  //    weights (that is all of them up to K = 16384; long rows with 2 MT units ahead instead:
+  //    12288 -> 3072 11.4 us for 10.4, 15360 -> 512 in chunks of two rows 18.8 for 17.6)
+  constexpr int XU = PIPED ? (MT == 1 ? 8 : 16) : (MT * B + 3) / 4;
+  auto x_load = [&](int u) __attribute__((always_inline)) {
+    const int r = u / ku, c = u - r * ku;
+    return buf_load16(xbuf, u < MT * ku && m0 + r < M ? (uint32_t)(((int64_t)(m0 + r) * ldx + 8 * c) * 2) : kOOB);
+  };
+  auto x_store = [&](int u, v4i v) __attribute__((always_inline)) {
+    const int r = u / ku, c = u - r * ku;
+    if (u < MT * ku) *(v4i*)(awq_lds + 16 * (r * ku + x_unit(c))) = v;
+  };
+  v4i xr[XU];
 #pragma unroll
-    for (int j = 0; j < AWQ_BATCH; ++j) {
+  for (int i = 0; i < XU; ++i) xr[i] = x_load(tid + i * AWQ_THREADS);
+
+  // 2. the first batch of weights, scales and zeros
+  struct Batch {
+    v4i wd[B];
+    uint16_t sc[B], ze[B];
+  };
+  auto load_batch = [&](Batch& bt, int s0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
       const bool ok = row_ok && (s0 + j) * AWQ_SPAN + 32 * t < K;
-      wd[j] = buf_load16(wbuf, ok ? wrow + (uint32_t)(AWQ_SPAN / 2) * (uint32_t)(s0 + j) : kOOB);
-      sc[j] = buf_load2(sbuf, ok ? grow + 16u * (uint32_t)(s0 + j) : kOOB);
-      ze[j] = buf_load2(zbuf, ok ? grow + 16u * (uint32_t)(s0 + j) : kOOB);
+      bt.sc[j] = buf_load2(sbuf, ok ? grow + 16u * (uint32_t)(s0 + j) : kOOB);
+      bt.ze[j] = buf_load2(zbuf, ok ? grow + 16u * (uint32_t)(s0 + j) : kOOB);
+      bt.wd[j] = buf_load16(wbuf, ok ? wrow + (uint32_t)(AWQ_SPAN / 2) * (uint32_t)(s0 + j) : kOOB);
     }
   };
-  // 1. the first batch of weights goes out before the activations are staged (its latency covers theirs)
-  load_batch(0);
+  Batch cur;
+  load_batch(cur, 0);
 
-  // 2. the MT activation rows into LDS (rows past M: zeros), units swizzled by x_unit
-  {
-    const rsrc_t xbuf = make_rsrc(x, (uint32_t)(((int64_t)(M - 1) * ldx + K) * 2));
-    for (int u = tid; u < MT * ku; u += AWQ_THREADS) {
-      const int r = u / ku, c = u - r * ku;
-      const v4i v = buf_load16(xbuf, m0 + r < M ? (uint32_t)(((int64_t)(m0 + r) * ldx + 8 * c) * 2) : kOOB);
-      *(v4i*)(awq_lds + 16 * (r * ku + x_unit(c))) = v;
-    }
-  }
-  __syncthreads();
+  // 3. the activations into LDS, units swizzled by x_unit
+#pragma unroll
+  for (int i = 0; i < XU; ++i) x_store(tid + i * AWQ_THREADS, xr[i]);
+  for (int u = tid + XU * AWQ_THREADS; u < MT * ku; u += AWQ_THREADS) x_store(u, x_load(u));
+  barrier_staged();
 
-  // 3. batches of spans: dequantize 32 codes, dot them with every activation row
+  // 4. batches of spans: dequantize 32 codes, dot them with every activation row
   float acc[MT];
 #pragma unroll
   for (int r = 0; r < MT; ++r) acc[r] = 0.0f;
-  for (int s0 = 0; s0 < spans; s0 += AWQ_BATCH) {
-    if (s0) load_batch(s0);
+  auto use_batch = [&](const Batch& bt, int s0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < AWQ_BATCH; ++j) {
-      if ((s0 + j) * AWQ_SPAN + 32 * t >= K) continue;  // past the row (K % 512 != 0)
-      const float sv = bf16_to_f32(sc[j]), zv = bf16_to_f32(ze[j]);
+    for (int j = 0; j < B; ++j) {
+      if ((s0 + j) * AWQ_SPAN + 32 * t >= K) continue;  // past the row (K % 512 != 0, or fewer spans)
+      const float sv = bf16_to_f32(bt.sc[j]), zv = bf16_to_f32(bt.ze[j]);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         uint32_t w[4];
-        dequant8((uint32_t)wd[j][q], sv, zv, w);
+        dequant8((uint32_t)bt.wd[j][q], sv, zv, w);
         const int unit = x_unit(64 * (s0 + j) + 4 * t + q);  // activation columns 512 s + 32 t + 8 q .. +8
 #pragma unroll
         for (int r = 0; r < MT; ++r) {
@@ -139,8 +169,19 @@ __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
         }
       }
     }
+  };
+  if (PIPED) {
+    Batch nxt;
+    for (int s0 = 0; s0 < spans; s0 += 2 * B) {
+      load_batch(nxt, s0 + B);  // past the row: no lane loads
+      use_batch(cur, s0);
+      load_batch(cur, s0 + 2 * B);
+      use_batch(nxt, s0 + B);
+    }
+  } else {
+    use_batch(cur, 0);
   }
-  // 4. team sum (lanes t ^ 8, 4, 2, 1), bias, bf16
+  // 5. team sum (lanes t ^ 8, 4, 2, 1), bias, bf16
   const float bv = (bias && row_ok) ? bf16_to_f32(bias[n]) : 0.0f;
 #pragma unroll
   for (int r = 0; r < MT; ++r) {
@@ -225,14 +266,24 @@ __global__ __launch_bounds__(256) void awq_w4a16_dequant_kernel(const uint32_t* 
   *(v4i*)(out + 8 * i) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
+// rows of up to AWQ_ALL spans load whole (three batch sizes, so that a short row does not issue loads for spans it does
+// not have)
 template <int MT>
 int launch_gemv(const void* x, int64_t ldx, const void* weight, const void* ws, const void* wz, const void* bias,
                 void* out, int64_t M, int64_t N, int64_t K, hipStream_t st) {
   const size_t lds = (size_t)MT * (size_t)K * 2;
+  const int64_t spans = (K + AWQ_SPAN - 1) / AWQ_SPAN;
   const dim3 grid((unsigned)((N + AWQ_TEAMS - 1) / AWQ_TEAMS), (unsigned)((M + MT - 1) / MT));
-  hipLaunchKernelGGL((awq_w4a16_gemv_kernel<MT>), grid, dim3(AWQ_THREADS), lds, st, (const uint16_t*)x, ldx,
-                     (const uint8_t*)weight, (const uint16_t*)ws, (const uint16_t*)wz, (const uint16_t*)bias,
-                     (uint16_t*)out, (int)M, (int)N, (int)K);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(AWQ_THREADS), lds, st, (const uint16_t*)x, ldx, (const uint8_t*)weight,
+                       (const uint16_t*)ws, (const uint16_t*)wz, (const uint16_t*)bias, (uint16_t*)out, (int)M, (int)N,
+                       (int)K);
+  };
+  if (spans > AWQ_ALL) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH, true>);
+  else if (spans > AWQ_BATCH + 2) go(awq_w4a16_gemv_kernel<MT, AWQ_ALL, false>);
+  else if (spans > AWQ_BATCH) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH + 2, false>);
+  else if (spans > AWQ_BATCH - 2) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH, false>);
+  else go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH - 2, false>);
   return gwa_check_launch("awq_w4a16_mm");
 }
 
@@ -268,8 +319,8 @@ extern "C" int gwa_awq_w4a16_mm(const void* x, int64_t ldx, const void* weight, 
               "%s: x must be 16-byte and weight 4-byte aligned", what);
   hipStream_t st = (hipStream_t)stream;
   // MFMA from 5 rows on (up to 4 the GEMV reads the weight once too, in whole 256-byte row segments: 5 rows at 3072 ->
-  // 18432 25.4 -> 17.9 us, 4 rows 16.4 -> 17.9), except long rows on few output rows: there the GEMV's chunks of rows
-  // are the parallelism (15360 -> 512, 16 rows: GEMV 19.5, MFMA 24.6; 15360 -> 1024 26.6 and 24.9; 8192 -> 512 16.3
+  // 18432 25.4 -> 17.9 us, 4 rows 15.8 -> 17.9), except long rows on few output rows: there the GEMV's chunks of rows
+  // are the parallelism (15360 -> 512, 16 rows: GEMV 17.7, MFMA 24.6; 15360 -> 1024 26 and 24.9; 8192 -> 512 16.3
   // and 13.9). 8 waves per workgroup for rows past 4096 inputs (15360 -> 2048, 16 rows: 4 waves 32.4, 8 25.0),
   // 4 otherwise (3072 -> 18432, 5 rows: 17.9 and 19.5).
   if (M > 4 && (N >= 1024 || K <= 8192)) {

@@ -53,6 +53,17 @@ def test_mm_matches_oracle(m, n, k, bias):
     check_output(y, ref, what=f"awq m={m} n={n} k={k} ({'gemv' if m <= AWQ_GEMV_MAX_M else 'dequant + gemm'})")
 
 
+@pytest.mark.parametrize("k", [1024, 1152, 2048, 2176, 3200, 4096, 4224, 8320, 15360])
+@pytest.mark.parametrize("m", [1, 2, 4])
+def test_mm_load_batches(m, k):
+    """Rows on both sides of each load batch (2, 4, 6 and 8 spans of 512 held at once, longer rows pipelined) and of
+    the activations requested ahead of the weights; N = 48 leaves no full multiple of 64 rows."""
+    codes, s, z, b, t = _layer(48, k, seed=m + k)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m + k)).to(torch.bfloat16)
+    y = torch.ops.cozy_gen_worker.awq_w4a16_mm(x.to(DEV), t["weight"], t["wscales"], t["wzeros"], t["bias"])
+    check_output(y, A.awq_linear(bits16(x), codes, s, z, b), what=f"awq m={m} k={k}")
+
+
 @pytest.mark.parametrize("m,n,k", [(5, 16, 128), (6, 48, 384), (8, 1008, 8192), (15, 1024, 4096), (16, 1024, 4224),
                                    (16, 32, 640), (9, 512, 8320), (16, 1008, 15360), (7, 1040, 15360)])
 def test_mm_several_rows(m, n, k):
