@@ -12,7 +12,7 @@
 //     kernel 1 (quant_g64.h quant8: smoothing by RN(1/s), scale RN(amax / 7), RNE codes), so codes and
 //     scales are bit-identical to kernel 1's; codes packed 8 nibbles per dword (element i at bits 4i..4i+3,
 //     the weight's packing), scales as floats, into LDS;
-//  2. sums kernel 1's la partial slots in slot order and rounds to bf16 (la_reduce_kernel's arithmetic);
+//  2. sums la's partial slots (svdq_la_few_rows_kernel below) in slot order and rounds to bf16 (la_reduce_kernel's arithmetic);
 //     (loaded in one batch: a dependent load per slot cost ~0.8 us each);
 //  3. P[m][row][g] = sum of the group's 64 code products (8 x v_dot8_i32_i4, exact) into LDS;
 //  4. one lane per (token, row) runs the output's chain in the GEMM's order: acc = fma(P_g, sx_g * sw_g, acc)
@@ -244,6 +244,37 @@ __global__ __launch_bounds__(GV_THREADS) void svdq_gemv_w4a4_kernel(
   }
 }
 
+// la partial slots for up to 16 rows: la_part[st][m][16 rb + r] = x[m, 128 st .. +128] . proj_down[.., 16 rb + r], the
+// products and order of kernel 1's slots (proj_down in its operand order, one stage per slot, so the sums are its
+// bits). One wave per stage and 16 ranks, operands straight into registers: 8 loads, 4 MFMAs, a store, nothing to share.
+// What bounds it is one memory latency and the launch; kernel 1, which this path ran for the slots alone, also quantizes
+// and stores records that nothing here reads: 16.1 -> 14.8 us for one token 3072 -> 18432 at rank 32, 17.9 -> 15.7 at
+// rank 128 (rank 0, without either: 10.5).
+template <int RB>
+__global__ __launch_bounds__(64) void svdq_la_few_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                              const uint16_t* __restrict__ pdo,
+                                                              float* __restrict__ la_part, int M, int K) {
+  constexpr int R = RB * 16;
+  const int lane = threadIdx.x, r = lane & 15, c = lane >> 4, st = blockIdx.x, rb = blockIdx.y;
+  const rsrc_t xbuf = make_rsrc(x, (uint32_t)(((int64_t)(M - 1) * ldx + K) * 2));
+  v4i xv[4], pv[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    xv[j] = buf_load16(xbuf, r < M ? (uint32_t)(((int64_t)r * ldx + 128 * st + 32 * c + 8 * j) * 2) : kOOB);
+    pv[j] = *(const v4i*)(pdo + ((((int64_t)st * 4 + j) * RB + rb) * 64 + lane) * 8);
+  }
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xv[j]), __builtin_bit_cast(v8bf, pv[j]), acc,
+                                                  0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = 4 * c + i;
+    if (m < M) la_part[((int64_t)st * M + m) * R + 16 * rb + r] = acc[i];
+  }
+}
+
 // activation records (+ 1 KB slack) and la partial slots of kernel 1, 256-byte aligned pieces
 int64_t records_bytes(int64_t M, int64_t K) { return ((K / 128) * M * GWA_FP6_REC + 1024 + 255) / 256 * 256; }
 
@@ -300,13 +331,25 @@ extern "C" int gwa_svdq_w4a4_linear_gemv(const void* x, int64_t ldx, const void*
   const float* la_part = nullptr;
   int P = 0;
   if (R > 0) {
-    // kernel 1 for la's partial slots (its records are not read: this path quantizes the rows itself)
-    uint8_t* ws = (uint8_t*)workspace;
-    float* part = (float*)(ws + records_bytes(M, K));
-    const int rc = gwa_svdq_quant_fp6(x, ldx, smooth, s2, proj_down_op6, R, ws, part, M, K, stream);
+    // la's partial slots, behind the records' place in the workspace (kernel 1's layout)
+    GWA_REQUIRE(GWA_ALIGNED(proj_down_op6, 16) && M * ldx * 2 < (1ll << 31),
+                "%s: proj_down_op6 must be 16-byte aligned and x below 2 GiB (buffer addressing)", what);
+    float* part = (float*)((uint8_t*)workspace + records_bytes(M, K));
+    P = (int)(K / 128);
+    const dim3 lgrid((unsigned)P, (unsigned)(R / 16));
+    const uint16_t *lx = (const uint16_t*)x, *pd = (const uint16_t*)proj_down_op6;
+#define GWA_LA_LAUNCH(RBV) \
+  hipLaunchKernelGGL((svdq_la_few_rows_kernel<RBV>), lgrid, dim3(64), 0, st, lx, ldx, pd, part, (int)M, (int)K)
+    switch (R) {
+      case 16: GWA_LA_LAUNCH(1); break;
+      case 32: GWA_LA_LAUNCH(2); break;
+      case 64: GWA_LA_LAUNCH(4); break;
+      default: GWA_LA_LAUNCH(8); break;
+    }
+#undef GWA_LA_LAUNCH
+    const int rc = gwa_check_launch(what);
     if (rc != GWA_OK) return rc;
     la_part = part;
-    P = (int)gwa_svdq_quant_fp6_partials(M, K, R);
   }
   // 32 rows per workgroup (half the workgroups: one round over the CUs at the modulation shapes) where the
   // items and LDS allow, else 16

@@ -161,3 +161,24 @@ def test_module_routes_small_m_and_graph_replays():
         with torch.no_grad():
             mod(x16)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("m,k,rank", [(1, 128, 16), (1, 3072, 32), (3, 640, 64), (4, 1024, 128), (8, 3072, 16),
+                                      (5, 2048, 32)])
+def test_low_rank_product_is_kernel_1s(m, k, rank):
+    """With zero codes and a one-hot proj_up an output is la itself: bit for bit the bf16 la of kernel 1 and its
+    reduction (the same products in the same order), strided rows included."""
+    from gen_worker_amd import ops
+
+    assert m <= ops.gemv_max_m(k, rank)
+    g = torch.Generator().manual_seed(m + k + rank)
+    x = torch.randn(m, k + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :k]
+    pd6 = ops.svdq_prep_proj_down_fp6((torch.randn(k, rank, generator=g) * 0.05).to(torch.bfloat16).to(DEV))
+    smooth = (torch.rand(k, generator=g) + 0.5).to(torch.bfloat16).to(DEV)
+    la = ops.svdq_quant_fp6(x.contiguous(), smooth, None, pd6)[1]
+    n = 2 * rank
+    up = torch.eye(rank, dtype=torch.bfloat16, device=DEV).repeat(2, 1)
+    y = ops.svdq_forward_gemv(x, smooth, None, pd6, torch.zeros(n, k // 2, dtype=torch.uint8, device=DEV),
+                              torch.ones(n, k // 64, dtype=torch.float16, device=DEV), None, up, None,
+                              torch.bfloat16, False)
+    assert np.array_equal(bits16(y), bits16(torch.cat([la, la], 1)))
