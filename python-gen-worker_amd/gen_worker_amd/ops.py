@@ -519,13 +519,10 @@ def linear_fp6_workspace_bytes(m: int, k: int, rank: int) -> int:
     return int(nat.load().gwa_svdq_w4a4_linear_fp6_workspace(m, k, rank))
 
 
-@torch.library.custom_op("cozy_gen_worker::svdq_forward_fp6", mutates_args=())
-def svdq_forward_fp6(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
-                     weight_fp6: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor], bias: Optional[Tensor],
-                     out_dtype: torch.dtype, gelu: bool) -> Tensor:
-    """The whole fp6-lane linear in one library call (``_SvdqFusedLinear.forward``, ``models/svdq_fused.py:516-527``):
-    kernel 1 into a workspace (records, la partial slots), the fixed-order la reduction and the GEMM with its
-    epilogue; bit-identical to ``svdq_quant_fp6`` followed by ``svdq_w4a4_linear_fp6``."""
+def _svdq_forward_fp6(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
+                      weight_fp6: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor], bias: Optional[Tensor],
+                      out_dtype: torch.dtype, gelu: bool) -> Tensor:
+    """The op ``svdq_forward_fp6`` without the dispatcher."""
     name = "svdq_forward_fp6"
     if x2.dim() != 2:
         raise SvdqOpError(f"{name}: x2 must be 2-D, got {tuple(x2.shape)}")
@@ -578,6 +575,16 @@ def svdq_forward_fp6(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor],
     return out
 
 
+@torch.library.custom_op("cozy_gen_worker::svdq_forward_fp6", mutates_args=())
+def svdq_forward_fp6(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
+                     weight_fp6: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor], bias: Optional[Tensor],
+                     out_dtype: torch.dtype, gelu: bool) -> Tensor:
+    """The whole fp6-lane linear in one library call (``_SvdqFusedLinear.forward``, ``models/svdq_fused.py:516-527``):
+    kernel 1 into a workspace (records, la partial slots), the fixed-order la reduction and the GEMM with its
+    epilogue; bit-identical to ``svdq_quant_fp6`` followed by ``svdq_w4a4_linear_fp6``."""
+    return _svdq_forward_fp6(x2, smooth, s2, proj_down_op6, weight_fp6, second, proj_up, bias, out_dtype, gelu)
+
+
 @svdq_forward_fp6.register_fake
 def _(x2, smooth, s2, proj_down_op6, weight_fp6, second, proj_up, bias, out_dtype, gelu):
     return x2.new_empty(int(x2.shape[0]), int(weight_fp6.shape[1]), dtype=out_dtype)
@@ -588,14 +595,10 @@ def gemv_max_m(k: int, rank: int) -> int:
     return int(nat.load().gwa_svdq_w4a4_gemv_max_m(k, rank))
 
 
-@torch.library.custom_op("cozy_gen_worker::svdq_forward_gemv", mutates_args=())
-def svdq_forward_gemv(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
-                      weight: Tensor, weight_scale: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor],
-                      bias: Optional[Tensor], out_dtype: torch.dtype, gelu: bool) -> Tensor:
-    """The whole linear for a few tokens (``_SvdqFusedLinear.forward``, ``models/svdq_fused.py:516-527``, at
-    M <= ``gemv_max_m``): the int4 weight [N, K/2] and its fp16 scales streamed once by a GEMV that quantizes
-    the rows with kernel 1's quantizer (bit-identical codes and scales) and sums kernel 1's la partial slots;
-    the group order and epilogue of the GEMM lane (only the low-rank sum rounds differently)."""
+def _svdq_forward_gemv(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
+                       weight: Tensor, weight_scale: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor],
+                       bias: Optional[Tensor], out_dtype: torch.dtype, gelu: bool) -> Tensor:
+    """The op ``svdq_forward_gemv`` without the dispatcher."""
     name = "svdq_forward_gemv"
     if x2.dim() != 2:
         raise SvdqOpError(f"{name}: x2 must be 2-D, got {tuple(x2.shape)}")
@@ -647,6 +650,18 @@ def svdq_forward_gemv(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor]
              _dt_code(out_dtype), nat.EPI_GELU_TANH if gelu else 0, m, n, k, nat.ptr(ws), int(ws.numel()),
              nat.stream_of(x2))
     return out
+
+
+@torch.library.custom_op("cozy_gen_worker::svdq_forward_gemv", mutates_args=())
+def svdq_forward_gemv(x2: Tensor, smooth: Optional[Tensor], s2: Optional[Tensor], proj_down_op6: Optional[Tensor],
+                      weight: Tensor, weight_scale: Tensor, second: Optional[Tensor], proj_up: Optional[Tensor],
+                      bias: Optional[Tensor], out_dtype: torch.dtype, gelu: bool) -> Tensor:
+    """The whole linear for a few tokens (``_SvdqFusedLinear.forward``, ``models/svdq_fused.py:516-527``, at
+    M <= ``gemv_max_m``): the int4 weight [N, K/2] and its fp16 scales streamed once by a GEMV that quantizes
+    the rows with kernel 1's quantizer (bit-identical codes and scales) and sums la's partial slots;
+    the group order and epilogue of the GEMM lane (only the low-rank sum rounds differently)."""
+    return _svdq_forward_gemv(x2, smooth, s2, proj_down_op6, weight, weight_scale, second, proj_up, bias,
+                              out_dtype, gelu)
 
 
 @svdq_forward_gemv.register_fake
@@ -731,7 +746,7 @@ class BoundLinearFp6:
     """One fp6-lane linear's resident operands bound for eager calls: the same library entry points and
     arguments as ``svdq_forward_fp6`` (and ``svdq_forward_gemv`` up to ``gemv_max_m`` tokens), so the output is
     the op's bit for bit, without the dispatcher's and the per-call operand checks' host time. The operands are
-    checked once, by running both ops on a 0-row activation; a call then checks only the activation (dtype,
+    checked once, by running both ops' bodies on a 0-row activation; a call then checks only the activation (dtype,
     device, width; rows with an unaligned stride are copied, as the op does), allocates the output and the
     workspace and enqueues on the current stream. The pointers are those of the tensors at binding: the owner
     rebinds when any of them changes (``key``), and the binding holds them (``held``). ``native`` is the same call
@@ -746,10 +761,10 @@ class BoundLinearFp6:
                  bias: Optional[Tensor], out_dtype: torch.dtype, gelu: bool, gemv_max_m: int) -> None:
         n = _fp6_records_k("BoundLinearFp6", weight_fp6, "weight_fp6")[0]
         x0 = torch.empty(0, k, dtype=torch.bfloat16, device=weight_fp6.device)
-        svdq_forward_fp6(x0, smooth, None, proj_down_op6, weight_fp6, second, proj_up, bias, out_dtype, gelu)
+        _svdq_forward_fp6(x0, smooth, None, proj_down_op6, weight_fp6, second, proj_up, bias, out_dtype, gelu)
         if gemv_max_m > 0:
-            svdq_forward_gemv(x0, smooth, None, proj_down_op6, weight, weight_scale, second, proj_up, bias, out_dtype,
-                              gelu)
+            _svdq_forward_gemv(x0, smooth, None, proj_down_op6, weight, weight_scale, second, proj_up, bias, out_dtype,
+                               gelu)
         if second is not None and second.dtype != torch.float32:
             raise SvdqOpError("BoundLinearFp6: second must be float32 (the op would convert it per call)")
         lib = nat.load()
@@ -1197,7 +1212,7 @@ class BoundLinearW8a8:
 # AWQ W4A16 (the adaLN modulation layers)
 # ---------------------------------------------------------------------------
 
-AWQ_GEMV_MAX_M = 16   # activation rows up to which the GEMV kernel runs; above, dequant + library GEMM
+AWQ_GEMV_MAX_M = 16   # activation rows up to which the HIP kernels run; above, dequant + library GEMM
 
 
 def _awq_check(name: str, weight: Tensor, wscales: Tensor, wzeros: Tensor, k: Optional[int]) -> tuple[int, int]:
@@ -1236,9 +1251,9 @@ def _(weight, wscales, wzeros):
 def awq_w4a16_mm(x2: Tensor, weight: Tensor, wscales: Tensor, wzeros: Tensor, bias: Optional[Tensor]) -> Tensor:
     """The reference's packed AWQ op (``models/svdq_awq_packed.py:48-115``, same name and schema):
     x2 bf16 [M, K], weight uint8 [N, K/2] (column 2j in the low nibble of byte j), wscales / wzeros bf16
-    [N, K/64], bias bf16 [N] or None -> bf16 [M, N]. Up to ``AWQ_GEMV_MAX_M`` rows run the HIP GEMV
-    (the weight read once per four rows); more rows dequantize the weight to bf16 once (HIP) and run a
-    library GEMM on it."""
+    [N, K/64], bias bf16 [N] or None -> bf16 [M, N]. Up to ``AWQ_GEMV_MAX_M`` rows run the HIP
+    kernels (up to 4 rows a GEMV, more an MFMA kernel: the weight read once); more rows dequantize the weight
+    to bf16 once (HIP) and run a library GEMM on it."""
     name = "awq_w4a16_mm"
     _check_dtype(name, x2, torch.bfloat16, what="x2")
     _check_dtype(name, bias, torch.bfloat16, what="bias")
