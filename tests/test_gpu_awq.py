@@ -82,6 +82,22 @@ def test_mm_several_rows(m, n, k):
     assert torch.equal(op(other, t["weight"], t["wscales"], t["wzeros"], t["bias"])[3], y[0])
 
 
+def test_c_entry_takes_more_than_16_rows():
+    """The C entry in chunks of 16 rows, the last one ragged, with a padded row stride: each chunk the op's bits."""
+    from gen_worker_amd import _native as nat
+
+    m, n, k, ld = 37, 48, 640, 648
+    _, _, _, _, t = _layer(n, k, seed=9)
+    x = torch.randn(m, ld, generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(DEV)
+    y = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    nat.call("gwa_awq_w4a16_mm", nat.ptr(x), ld, nat.ptr(t["weight"]), nat.ptr(t["wscales"]), nat.ptr(t["wzeros"]),
+             nat.ptr(t["bias"]), nat.ptr(y), m, n, k, nat.stream_of(x))
+    op = torch.ops.cozy_gen_worker.awq_w4a16_mm
+    for r0 in (0, 16, 32):
+        xc = x[r0:r0 + 16, :k].contiguous()
+        assert torch.equal(op(xc, t["weight"], t["wscales"], t["wzeros"], t["bias"]), y[r0:r0 + 16])
+
+
 def test_mm_deterministic_and_row_independent():
     """Repeated calls agree bit for bit, and a row's result does not depend on the other rows of its chunk."""
     _, _, _, _, t = _layer(1024, 3072, seed=3)
