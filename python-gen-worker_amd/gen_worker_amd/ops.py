@@ -1094,12 +1094,8 @@ def _(qa, qw):
 # W8A8
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("cozy_gen_worker::w8a8_quant", mutates_args=())
-def w8a8_quant(x2: Tensor, pertensor: bool = False, static: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
-    """int8 activation quant in the modes of the reference's ``quantize(x2, pertensor, static)``
-    (``models/w8a8.py:261-273``): ``static`` (the layer's ``input_scale`` [1, 1] fp32) is used unchanged,
-    as ``sa`` [1, 1] when ``pertensor`` else expanded to [M, 1]; without it ``sa`` is ``max(amax/127, 1e-12)``
-    over the whole tensor ([1, 1]) or per token ([M, 1]). Returns (q int8 [M, K], sa)."""
+def _w8a8_quant(x2: Tensor, pertensor: bool = False, static: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
+    """The op ``w8a8_quant`` without the dispatcher."""
     name = "w8a8_quant"
     _check_dtype(name, x2, torch.bfloat16, what="x2")
     _check_dtype(name, static, torch.float32, what="static")
@@ -1115,17 +1111,24 @@ def w8a8_quant(x2: Tensor, pertensor: bool = False, static: Optional[Tensor] = N
     return q, sa
 
 
+@torch.library.custom_op("cozy_gen_worker::w8a8_quant", mutates_args=())
+def w8a8_quant(x2: Tensor, pertensor: bool = False, static: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
+    """int8 activation quant in the modes of the reference's ``quantize(x2, pertensor, static)``
+    (``models/w8a8.py:261-273``): ``static`` (the layer's ``input_scale`` [1, 1] fp32) is used unchanged,
+    as ``sa`` [1, 1] when ``pertensor`` else expanded to [M, 1]; without it ``sa`` is ``max(amax/127, 1e-12)``
+    over the whole tensor ([1, 1]) or per token ([M, 1]). Returns (q int8 [M, K], sa)."""
+    return _w8a8_quant(x2, pertensor, static)
+
+
 @w8a8_quant.register_fake
 def _(x2, pertensor=False, static=None):
     m, k = int(x2.shape[0]), int(x2.shape[1])
     return x2.new_empty(m, k, dtype=torch.int8), x2.new_empty(1 if pertensor else m, 1, dtype=torch.float32)
 
 
-@torch.library.custom_op("cozy_gen_worker::w8a8_scaled_mm", mutates_args=())
-def w8a8_scaled_mm(qa: Tensor, weight: Tensor, sa: Tensor, weight_scale: Tensor, bias: Optional[Tensor],
-                   out_dtype: torch.dtype) -> Tensor:
-    """``_scaled_mm(qa, weight.t(), scale_a=sa, scale_b=weight_scale.t(), bias, out_dtype)`` on int8 codes;
-    ``sa`` holds one scale per row ([M, 1], rowwise) or one for the tensor ([1, 1], pertensor)."""
+def _w8a8_scaled_mm(qa: Tensor, weight: Tensor, sa: Tensor, weight_scale: Tensor, bias: Optional[Tensor],
+                    out_dtype: torch.dtype) -> Tensor:
+    """The op ``w8a8_scaled_mm`` without the dispatcher."""
     name = "w8a8_scaled_mm"
     _check_dtype(name, qa, torch.int8, what="qa")
     _check_dtype(name, weight, torch.int8, what="weight")
@@ -1149,6 +1152,14 @@ def w8a8_scaled_mm(qa: Tensor, weight: Tensor, sa: Tensor, weight_scale: Tensor,
     return out
 
 
+@torch.library.custom_op("cozy_gen_worker::w8a8_scaled_mm", mutates_args=())
+def w8a8_scaled_mm(qa: Tensor, weight: Tensor, sa: Tensor, weight_scale: Tensor, bias: Optional[Tensor],
+                   out_dtype: torch.dtype) -> Tensor:
+    """``_scaled_mm(qa, weight.t(), scale_a=sa, scale_b=weight_scale.t(), bias, out_dtype)`` on int8 codes;
+    ``sa`` holds one scale per row ([M, 1], rowwise) or one for the tensor ([1, 1], pertensor)."""
+    return _w8a8_scaled_mm(qa, weight, sa, weight_scale, bias, out_dtype)
+
+
 @w8a8_scaled_mm.register_fake
 def _(qa, weight, sa, weight_scale, bias, out_dtype):
     return qa.new_empty(int(qa.shape[0]), int(weight.shape[0]), dtype=out_dtype)
@@ -1157,8 +1168,8 @@ def _(qa, weight, sa, weight_scale, bias, out_dtype):
 class BoundLinearW8a8:
     """A W8A8 linear's resident operands bound for eager calls: ``w8a8_quant`` then ``w8a8_scaled_mm`` as the
     ops enqueue them (same entry points and arguments, so the same output bit for bit) without the dispatcher
-    and the per-call operand checks. The operands are checked once by both ops on a 0-row activation; a call
-    checks the activation (bf16, contiguous [M, K] on this device) and allocates the codes, the activation
+    and the per-call operand checks. The operands are checked once by both ops' bodies on a 0-row activation; a
+    call checks the activation (bf16, contiguous [M, K] on this device) and allocates the codes, the activation
     scales and the output. The owner rebinds when an operand changes (``key``); the binding holds the tensors
     whose pointers it uses (``held``). ``native`` is the same call in native code, which the owner tries first."""
 
@@ -1169,8 +1180,8 @@ class BoundLinearW8a8:
                  static: Optional[Tensor], pertensor: bool, out_dtype: torch.dtype) -> None:
         n, k = int(weight.shape[0]), int(weight.shape[1])
         x0 = torch.empty(0, k, dtype=torch.bfloat16, device=weight.device)
-        q0, sa0 = w8a8_quant(x0, pertensor, static)
-        w8a8_scaled_mm(q0, weight, sa0, weight_scale, bias, out_dtype)
+        q0, sa0 = _w8a8_quant(x0, pertensor, static)
+        _w8a8_scaled_mm(q0, weight, sa0, weight_scale, bias, out_dtype)
         lib = nat.load()
         self.key, self.held, self.native = key, held, None
         self.device = weight.device
