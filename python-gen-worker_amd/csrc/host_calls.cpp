@@ -13,6 +13,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
 
@@ -187,12 +188,13 @@ bool still_bound(const BoundCall* b, PyObject* dict) {
   return true;
 }
 
-// A plain tensor in plain eager mode: what ops.eager_call_ok asks, and no wrapper that hides a storage
+// A plain tensor in plain eager mode: what ops.eager_call_ok asks, and no wrapper that hides a storage. A trace (which
+// sets no mode) records operators: it would hold what is computed beside them as a constant.
 bool plain_call(const Tensor& x) {
   if (!x.is_cuda() || x.layout() != at::kStrided || !x.has_storage()) return false;
   if (x.requires_grad() && at::GradMode::is_enabled()) return false;
   if (c10::impl::TorchDispatchModeTLS::stack_len() != 0) return false;
-  if (at::impl::torch_function_mode_enabled()) return false;
+  if (at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing()) return false;
   return !x.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
                                                    c10::DispatchKey::FuncTorchBatched,
                                                    c10::DispatchKey::FuncTorchGradWrapper,

@@ -213,3 +213,36 @@ def test_quantizer_without_a_low_rank_product_equals_the_oracle(m, k, smooth):
         nat.call("gwa_svdq_quant_int4", a.data_ptr(), a.stride(0), nat.ptr(smd), one.data_ptr(), None, 0, nat.QFMT_INT4,
                  q.data_ptr(), s.data_ptr(), None, m, k, nat.stream_of(a))
         assert np.array_equal(q.cpu().numpy(), want_q) and np.array_equal(bits(s.cpu()), want_s.view(np.uint16))
+
+
+def _layer(kind, n=272, k=448):
+    from gen_worker_amd import synthetic
+    from gen_worker_amd.svdq import build_svdq_w4a4_linear
+    from gen_worker_amd.w8a8 import build_int8_linear
+
+    if kind == "awq":
+        return _awq(n, 384), 384
+    if kind == "w8a8":
+        w8 = synthetic.w8a8_layer(n, k)
+        return build_int8_linear(qweight=w8.qweight, weight_scale=w8.weight_scale, bias=w8.bias, device=DEV), k
+    k = 512 if kind == "w4a4_gemv" else k
+    _, layer = _operands(4, n, k, 32)
+    return build_svdq_w4a4_linear(qweight=layer.qweight, wscales=layer.wscales, smooth=layer.smooth,
+                                  proj_down=layer.proj_down, proj_up=layer.proj_up, bias=layer.bias, device=DEV), k
+
+
+KINDS = ["w4a4", "w4a4_gemv", "w8a8", "awq"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_trace_records_the_operators(kind):
+    """A traced layer computes its output from its input: the native call, which a trace cannot see, leaves the traced
+    call to the operators."""
+    mod, k = _layer(kind)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a, b = (torch.randn(4, k, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    with torch.no_grad():
+        mod(a)   # the native call is bound
+        traced = torch.jit.trace(mod, (a,))
+        assert "cozy_gen_worker" in str(traced.inlined_graph)
+        assert _same(traced(a), mod(a)) and _same(traced(b), mod(b))
