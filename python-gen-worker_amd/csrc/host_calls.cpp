@@ -189,13 +189,15 @@ bool still_bound(const BoundCall* b, PyObject* dict) {
 }
 
 // A plain tensor in plain eager mode: what ops.eager_call_ok asks, and no wrapper that hides a storage. A trace (which
-// sets no mode) records operators: it would hold what is computed beside them as a constant.
+// sets no mode) records operators: it would hold what is computed beside them as a constant. A lazily negated tensor's
+// storage holds the values before the negation, which the dispatcher carries out ahead of an operator.
 bool plain_call(const Tensor& x) {
   if (!x.is_cuda() || x.layout() != at::kStrided || !x.has_storage()) return false;
   if (x.requires_grad() && at::GradMode::is_enabled()) return false;
   if (c10::impl::TorchDispatchModeTLS::stack_len() != 0) return false;
   if (at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing()) return false;
   return !x.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
+                                                   c10::DispatchKey::Negative, c10::DispatchKey::Conjugate,
                                                    c10::DispatchKey::FuncTorchBatched,
                                                    c10::DispatchKey::FuncTorchGradWrapper,
                                                    c10::DispatchKey::ZeroTensor}));

@@ -246,3 +246,12 @@ def test_a_trace_records_the_operators(kind):
         traced = torch.jit.trace(mod, (a,))
         assert "cozy_gen_worker" in str(traced.inlined_graph)
         assert _same(traced(a), mod(a)) and _same(traced(b), mod(b))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_lazily_negated_activation_is_negated(kind):
+    mod, k = _layer(kind)
+    x = torch.randn(4, k, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV).to(torch.bfloat16)
+    want = mod((-x).contiguous())
+    lazy = torch._neg_view(x)
+    assert lazy.is_neg() and _same(mod(lazy), want)
