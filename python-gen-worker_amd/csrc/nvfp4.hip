@@ -130,9 +130,12 @@ __device__ __forceinline__ float nvfp4_dynamic_s2(const float* __restrict__ part
 // in the last place is exact in one fma, and the correction's own error is below 2^-23 of such a unit); + 0 makes the
 // quotient of -0 a +0, whose sign bit the reference leaves clear. The hardware's conversion (round to nearest even,
 // saturating at 6) then is the reference's count of bounds and tie bumps but for the ties 2.5 and 3.5, which the
-// reference takes to 3. A wave whose den or mb is no ordinary number takes the reference's own steps.
+// reference takes to 3. A wave whose den or mb is no ordinary number, or whose quotient may pass 2^100 (past 2^128 the
+// residual of an infinite quotient would be NaN; only a static s2 far below the data comes near), takes the reference's
+// own steps.
 __device__ __forceinline__ uint32_t e2m1_codes8(const float (&v)[8], float den, uint32_t mb) {
-  const bool plain = den >= 0x1p-60f && den <= 0x1p16f && mb < 0x7F800000u;
+  // mb as a float: the comparison is false for a NaN, and den * 2^100 is finite for these den
+  const bool plain = den >= 0x1p-60f && den <= 0x1p16f && __uint_as_float(mb) <= den * 0x1p100f;
   uint32_t codes = 0;
   if (__builtin_expect(__any(!plain), 0)) {
 #pragma unroll 1

@@ -241,3 +241,23 @@ def test_scale_bias_tile_ends(m, n):
     torch.ops.cozy_gen_worker.nvfp4_scale_bias(yd, torch.tensor(s2, device=DEV), torch.tensor(ws2, device=DEV), _bf16(b))
     want = N.bf16_round(N.bf16_round(y * N.bf16_round(s2 * ws2)) + b)
     assert np.array_equal(yd.float().cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("s2v", [2.0 ** -10, 1e-12, 2.0 ** -60, 1e-20])
+def test_quotients_past_the_float_range_saturate(s2v):
+    """A static second scale far below the data: the block scales clamp at 448 and the quotients pass 2^128, where the
+    division gives an infinity and the code of +-6; zeros and small values of the same block keep theirs."""
+    s2v = np.float32(s2v)
+    x = np.zeros((4, 64), np.float32)
+    x[0, ::2], x[0, 1::2] = 3e38, -3e38
+    x[1, 0], x[1, 1], x[1, 2] = -3.3e38, 448 * s2v, -1e30
+    x[2, :16], x[2, 16:32] = -1e35, 2.0 ** 100 * 448 * s2v
+    x[3, 5], x[3, 40] = -1e38, 2.0 ** 60
+    x = N.bf16_round(x)
+    cg = torch.ops.cozy_gen_worker
+    q, sc, xdq = cg.nvfp4_quant_act(_bf16(x), torch.tensor(s2v, device=DEV), False, True)
+    with np.errstate(over="ignore"):
+        oq, osc = N.quantize_activation(x, s2v)
+    assert np.array_equal(sc.cpu().numpy(), osc) and np.array_equal(q.cpu().numpy(), oq)
+    assert np.array_equal(xdq.float().cpu().numpy().view(np.uint32), N.dequantize(oq, osc).view(np.uint32))
+    assert torch.equal(cg.nvfp4_act_values(_bf16(x), torch.tensor(s2v, device=DEV))[0], xdq)
