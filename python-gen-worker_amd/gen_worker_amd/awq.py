@@ -344,8 +344,8 @@ class AwqPackedLinear(nn.Module):
     def forward(self, x: Tensor) -> Tensor:
         native = ops.awq_native()
         if native is not None and not torch.compiler.is_compiling():
-            b = self._buffers
-            y = native(x, b["weight"], b["wscales"], b["wzeros"], self.bias, ops.AWQ_GEMV_MAX_M)
+            b = self._buffers.get   # an operand kept elsewhere (a Parameter, a parametrization) is the operator's to read
+            y = native(x, b("weight"), b("wscales"), b("wzeros"), self.bias, ops.AWQ_GEMV_MAX_M)
             if y is not None:
                 return y
         lead = x.shape[:-1]

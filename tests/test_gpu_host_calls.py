@@ -255,3 +255,28 @@ def test_a_lazily_negated_activation_is_negated(kind):
     want = mod((-x).contiguous())
     lazy = torch._neg_view(x)
     assert lazy.is_neg() and _same(mod(lazy), want)
+
+
+@pytest.mark.parametrize("how", ["parameter", "attribute", "parametrized"])
+def test_awq_layer_serves_operands_that_are_not_buffers(how):
+    import torch.nn.utils.parametrize as P
+
+    mod = _awq(144, 384)
+    x = torch.randn(3, 384, generator=torch.Generator(device=DEV).manual_seed(7), device=DEV).to(torch.bfloat16)
+    want = mod(x)
+    w = mod.weight
+    if how == "parameter":
+        del mod.weight
+        mod.weight = torch.nn.Parameter(w, requires_grad=False)
+    elif how == "attribute":
+        del mod.weight
+        mod.weight = w
+    else:
+        class Flip(torch.nn.Module):
+            def forward(self, t):
+                return t ^ 0xFF
+
+        with torch.no_grad():
+            mod.weight.copy_(w ^ 0xFF)
+            P.register_parametrization(mod, "weight", Flip())
+    assert "weight" not in mod._buffers and _same(mod(x), want)
