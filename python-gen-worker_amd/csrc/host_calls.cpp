@@ -188,19 +188,22 @@ bool still_bound(const BoundCall* b, PyObject* dict) {
   return true;
 }
 
-// A plain tensor in plain eager mode: what ops.eager_call_ok asks, and no wrapper that hides a storage. A trace (which
-// sets no mode) records operators: it would hold what is computed beside them as a constant. A lazily negated tensor's
-// storage holds the values before the negation, which the dispatcher carries out ahead of an operator.
+// Keys under which the dispatcher does something to an operand ahead of an operator's CUDA kernel: a wrapper that hides
+// its storage, or a lazy negation, whose storage holds the values before it
+constexpr c10::DispatchKeySet kNotPlain({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
+                                         c10::DispatchKey::Negative, c10::DispatchKey::Conjugate,
+                                         c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::ZeroTensor});
+bool plain_tensor(const Tensor& t) {
+  return !(t.requires_grad() && at::GradMode::is_enabled()) && !t.key_set().has_any(kNotPlain);
+}
+
+// A plain tensor in plain eager mode: what ops.eager_call_ok asks. A trace (which sets no mode) records operators: it
+// would hold what is computed beside them as a constant.
 bool plain_call(const Tensor& x) {
-  if (!x.is_cuda() || x.layout() != at::kStrided || !x.has_storage()) return false;
-  if (x.requires_grad() && at::GradMode::is_enabled()) return false;
-  if (c10::impl::TorchDispatchModeTLS::stack_len() != 0) return false;
-  if (at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing()) return false;
-  return !x.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Functionalize,
-                                                   c10::DispatchKey::Negative, c10::DispatchKey::Conjugate,
-                                                   c10::DispatchKey::FuncTorchBatched,
-                                                   c10::DispatchKey::FuncTorchGradWrapper,
-                                                   c10::DispatchKey::ZeroTensor}));
+  return plain_tensor(x) && x.is_cuda() && x.layout() == at::kStrided && x.has_storage() &&
+         c10::impl::TorchDispatchModeTLS::stack_len() == 0 && !at::impl::torch_function_mode_enabled() &&
+         !torch::jit::tracer::isTracing();
 }
 
 // the output of a layer for x [..., k]: x's leading dimensions and n columns
@@ -318,15 +321,15 @@ bool awq_fits(const Tensor& weight, const Tensor& wscales, const Tensor& wzeros,
 PyObject* awq_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs != 6 || !g_bound || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
-  for (int i = 1; i < 4; ++i)
-    if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
-  if (args[4] != Py_None && !THPVariable_Check(args[4])) Py_RETURN_NONE;
+  for (int i = 1; i < 5; ++i)  // operands that a subclass, autograd or a transform has a say in are the operator's
+    if (!(i == 4 && args[i] == Py_None) &&
+        (!THPVariable_CheckExact(args[i]) || !plain_tensor(THPVariable_Unpack(args[i]))))
+      Py_RETURN_NONE;
   const Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &sc = THPVariable_Unpack(args[2]),
                &z = THPVariable_Unpack(args[3]);
   OptTensor bias;
   if (args[4] != Py_None) bias = THPVariable_Unpack(args[4]);
   const int64_t k = w.dim() == 2 ? w.size(1) * 2 : 0, m = plain_rows(x, k);
-  if (bias.has_value() && bias->requires_grad() && at::GradMode::is_enabled()) Py_RETURN_NONE;
   if (m == 0 || m > PyLong_AsLongLong(args[5]) || !awq_fits(w, sc, z, bias, x.device(), k)) Py_RETURN_NONE;
   Tensor out;
   int rc;

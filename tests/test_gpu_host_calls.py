@@ -280,3 +280,33 @@ def test_awq_layer_serves_operands_that_are_not_buffers(how):
             mod.weight.copy_(w ^ 0xFF)
             P.register_parametrization(mod, "weight", Flip())
     assert "weight" not in mod._buffers and _same(mod(x), want)
+
+
+class _Seen(torch.Tensor):
+    calls: list = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.calls.append(str(func))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+def test_awq_layer_leaves_operands_the_operator_has_to_see():
+    """A weight that vmap batches, a scale that autograd follows, and an operand of a tensor subclass go through the
+    operator as before."""
+    mod = _awq(144, 384)
+    x = torch.randn(3, 384, generator=torch.Generator(device=DEV).manual_seed(7), device=DEV).to(torch.bfloat16)
+    want = mod(x)
+    both = torch.stack([mod.weight, mod.weight ^ 0x55])
+    got = torch.vmap(lambda w: torch.func.functional_call(mod, {"weight": w}, (x,)))(both)
+    assert _same(got[0], want)
+    assert _same(got[1], torch.func.functional_call(mod, {"weight": both[1].clone()}, (x,)))
+    mod.wscales.requires_grad_()
+    assert mod(x).requires_grad and _same(mod(x).detach(), want)
+    with torch.no_grad():
+        assert not mod(x).requires_grad
+    mod.wscales.requires_grad_(False)
+    mod.wzeros = mod.wzeros.as_subclass(_Seen)
+    _Seen.calls.clear()
+    assert _same(mod(x).as_subclass(torch.Tensor), want)
+    assert any("awq_w4a16_mm" in c for c in _Seen.calls), _Seen.calls
