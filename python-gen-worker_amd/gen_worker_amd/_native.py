@@ -2,7 +2,8 @@
 
 The library is located next to this file, or at ``$GEN_WORKER_AMD_LIB``.
 There is no fallback: a missing or unloadable library raises
-:class:`NativeUnavailable`, and every failed call raises
+:class:`NativeUnavailable` (the native host calls beside it are optional: they
+only make the same calls in less host time), and every failed call raises
 :class:`NativeError` with the library's own message (the equivalents of the
 ``TORCH_CHECK`` / launch-check failures of ``csrc/cozy_kernels/probe.cu:15-25``
 in the reference).
@@ -13,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 from typing import Optional
 
@@ -172,9 +174,10 @@ def load() -> ctypes.CDLL:
             from . import ops
 
             ops.bind_host_calls(lib)
-        except ImportError as exc:
-            raise NativeUnavailable(f"the native host calls failed to load (build them with `python -m "
-                                    f"gen_worker_amd.build`): {exc}") from exc
+        except ImportError as exc:   # every call they serve has a Python path to the same entry points
+            warnings.warn(f"gen_worker_amd: eager calls are made from Python, at more host time a call: the native "
+                          f"host calls did not load (`python -m gen_worker_amd.build` builds them): {exc}",
+                          RuntimeWarning, stacklevel=2)
         _lib = lib
         return lib
 

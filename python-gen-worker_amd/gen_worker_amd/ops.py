@@ -690,25 +690,27 @@ def bind_host_calls(lib) -> None:
     addresses = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in nat.EXPORTED_SYMBOLS}
     bodies = {"svdq_quant": _svdq_quant_body, "svdq_gemm_w4a4_lora": _svdq_gemm_w4a4_lora_body}
     _host_calls.bind(addresses, bodies, _REF_WEIGHT_FP6.get)
-    global _awq_native
-    _awq_native = _host_calls.awq_forward
+    global _host, _awq_native
+    _host, _awq_native = _host_calls, _host_calls.awq_forward
 
 
-_awq_native = None   # the AWQ layer's native call, once the library is loaded
+_host = None         # the native host calls, once they are bound
+_awq_native = None   # the AWQ layer's, likewise
 
 
 def awq_native():
     """``(x, weight, wscales, wzeros, bias, max_rows) -> output``, or None where ``awq_w4a16_mm`` has to decide (every
-    operand is checked on each call); None before the library is loaded."""
+    operand is checked on each call); None before the library is loaded and without the native host calls."""
     return _awq_native
 
 
 def _native_call(kind: int, mod, names: tuple, operands: tuple, versions: tuple, out_dtype: torch.dtype, k: int,
                  n: int, rank: int, gemv_max_m: int, flags: int):
     """A native bound call for ``mod``: good while each of ``names`` is the object it is now and each operand keeps
-    its storage (and version, where one is given); None for a module that keeps one of them elsewhere."""
-    from . import _host_calls
-
+    its storage (and version, where one is given); None for a module that keeps one of them elsewhere, and without
+    the native host calls."""
+    if _host is None:
+        return None
     attrs = []
     for name in names:
         for where, d in enumerate((mod.__dict__, mod._buffers, mod._parameters)):
@@ -717,7 +719,7 @@ def _native_call(kind: int, mod, names: tuple, operands: tuple, versions: tuple,
                 break
         else:
             return None
-    return _host_calls.BoundCall(kind, attrs, list(operands), list(versions), out_dtype, k, n, rank, gemv_max_m, flags)
+    return _host.BoundCall(kind, attrs, list(operands), list(versions), out_dtype, k, n, rank, gemv_max_m, flags)
 
 
 def native_w4a4(mod, out_dtype: torch.dtype, gelu: bool):

@@ -310,3 +310,20 @@ def test_awq_layer_leaves_operands_the_operator_has_to_see():
     _Seen.calls.clear()
     assert _same(mod(x).as_subclass(torch.Tensor), want)
     assert any("awq_w4a16_mm" in c for c in _Seen.calls), _Seen.calls
+
+
+def test_layers_without_the_native_host_calls(monkeypatch):
+    """What ``_native.load`` leaves where the extension does not import: the same bits from the Python paths."""
+    from gen_worker_amd import ops
+
+    for kind in KINDS:
+        mod, k = _layer(kind)
+        x = torch.randn(4, k, generator=torch.Generator(device=DEV).manual_seed(11), device=DEV).to(torch.bfloat16)
+        mod(x)
+        want = mod(x)
+        with monkeypatch.context() as mp:
+            mp.setattr(ops, "_host", None)
+            mp.setattr(ops, "_awq_native", None)
+            mod._bound = None
+            assert _same(mod(x), want) and _same(mod(x), want), kind
+            assert mod._bound is None or mod._bound.native is None

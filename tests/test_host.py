@@ -54,6 +54,41 @@ def test_debug_build_exports_the_header_and_the_release_build_refuses_its_query(
     assert "debug" in dbg.gwa_build_info().decode()
 
 
+def _fresh_load(before: str) -> str:
+    """Output of a process that runs ``before``, then loads the library and prints the warnings of it and whether the
+    native host calls are bound."""
+    import subprocess
+    import sys
+
+    code = f"""
+import sys, warnings
+sys.path.insert(0, {str(ROOT / "python-gen-worker_amd")!r})
+{before}
+import torch
+from gen_worker_amd import _native, ops
+with warnings.catch_warnings(record=True) as w:
+    warnings.simplefilter("always")
+    lib = _native.load()
+print("loaded", lib.gwa_version(), "bound", ops.awq_native() is not None, ops._host is not None)
+print([str(x.message) for x in w])
+try:
+    torch.ops.cozy_gen_worker.svdq_quant(torch.zeros(2, 64, dtype=torch.bfloat16), None, torch.ones(()), False)
+except ops.SvdqOpError as e:
+    print("op", e)
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stderr
+    return res.stdout
+
+
+def test_library_loads_without_the_native_host_calls():
+    """Another Python or torch than they were built for leaves the Python paths in place, with a warning."""
+    out = _fresh_load("")
+    assert "loaded 1 bound True True" in out and "[]" in out and "op svdq_quant" in out
+    out = _fresh_load("sys.modules['gen_worker_amd._host_calls'] = None")
+    assert "loaded 1 bound False False" in out and "host calls did not load" in out and "op svdq_quant" in out
+
+
 def test_library_is_a_gfx950_code_object():
     from gen_worker_amd import _native
 
