@@ -71,8 +71,14 @@ enum { GWA_FP6_REC = 104 };
  * records plus this slack with GWA_ERR_INVALID. */
 enum { GWA_FP6_RECORD_SLACK = 1024 };
 
-/* Library version and build description ("archs=gfx950 hip=..."). Mirrors
- * cozy_kernels::build_info, csrc/cozy_kernels/ops.cpp:23-27. */
+/* Version of this interface: raised when an entry point's arguments or their
+ * meaning change. A caller compiled against this header that resolves the
+ * entry points at run time compares it with gwa_version() first. */
+enum { GWA_VERSION = 1 };
+
+/* Library version (the GWA_VERSION it was built with) and build description
+ * ("archs=gfx950 hip=..."). Mirrors cozy_kernels::build_info,
+ * csrc/cozy_kernels/ops.cpp:23-27. */
 int gwa_version(void);
 const char* gwa_build_info(void);
 

@@ -26,7 +26,7 @@ int gwa_check_launch(const char* what) {
   return GWA_OK;
 }
 
-extern "C" int gwa_version(void) { return 1; }
+extern "C" int gwa_version(void) { return GWA_VERSION; }
 
 extern "C" const char* gwa_build_info(void) {
   static char buf[256];

@@ -16,6 +16,7 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
+#include <torch/version.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
 
@@ -486,5 +487,8 @@ PyMODINIT_FUNC PyInit__host_calls() {
   if (!m) return nullptr;
   Py_INCREF(&BoundType);
   if (PyModule_AddObject(m, "BoundCall", (PyObject*)&BoundType) < 0) return nullptr;
+  // what this was compiled against: compared with the library's and torch's own before anything is bound
+  if (PyModule_AddIntConstant(m, "GWA_VERSION", GWA_VERSION) < 0) return nullptr;
+  if (PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION) < 0) return nullptr;
   return m;
 }

@@ -682,11 +682,17 @@ def eager_call_ok(x2: Tensor) -> bool:
 
 def bind_host_calls(lib) -> None:
     """Give the native host calls (``csrc/host_calls.cpp``) the loaded library's entry points and the Python bodies
-    they hand back to; from then on ``svdq_quant`` and ``svdq_gemm_w4a4_lora`` run their native CUDA kernels."""
+    they hand back to; from then on ``svdq_quant`` and ``svdq_gemm_w4a4_lora`` run their native CUDA kernels.
+    ImportError where they are not there, or were compiled against another interface or torch than these."""
     import ctypes
 
     from . import _host_calls
 
+    built = (_host_calls.GWA_VERSION, _host_calls.TORCH_VERSION)
+    here = (lib.gwa_version(), torch.__version__.split("+")[0])
+    if built != here:
+        raise ImportError(f"they were built for interface {built[0]} and torch {built[1]}, this is {here[0]} and "
+                          f"{here[1]}")
     addresses = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in nat.EXPORTED_SYMBOLS}
     bodies = {"svdq_quant": _svdq_quant_body, "svdq_gemm_w4a4_lora": _svdq_gemm_w4a4_lora_body}
     _host_calls.bind(addresses, bodies, _REF_WEIGHT_FP6.get)

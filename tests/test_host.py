@@ -89,6 +89,13 @@ def test_library_loads_without_the_native_host_calls():
     assert "loaded 1 bound False False" in out and "host calls did not load" in out and "op svdq_quant" in out
 
 
+@pytest.mark.parametrize("name,value", [("GWA_VERSION", 0), ("TORCH_VERSION", "1.0.0")])
+def test_host_calls_built_for_another_interface_or_torch_are_not_bound(name, value):
+    """The extension calls the library through bare addresses: it is bound only to the header it was compiled with."""
+    out = _fresh_load(f"import torch\nfrom gen_worker_amd import _host_calls\n_host_calls.{name} = {value!r}")
+    assert "loaded 1 bound False False" in out and "were built for" in out and "op svdq_quant" in out
+
+
 def test_library_is_a_gfx950_code_object():
     from gen_worker_amd import _native
 
