@@ -376,9 +376,9 @@ int64_t gwa_svdq_w4a4_linear_fp6_noalloc_scratch_bytes(void);
  * would spend 32-128 rows of work on each real one. Streams the int4 weight
  * in the reference's layout (the module's `weight` uint8 [N, K/2], two's-
  * complement nibbles, low nibble = even input; `weight_scale` fp16 [N, K/64])
- * once; kernel 1 (gwa_svdq_quant_fp6) supplies la's partial slots when rank >
- * 0, and the GEMV quantizes the rows itself with kernel 1's quantizer (codes
- * and scales bit-identical). Same group order and epilogue as the GEMM
+ * once; la's partial slots (when rank > 0) come from a kernel of their own, one
+ * slot per 128 inputs, and the GEMV quantizes the rows itself with kernel 1's
+ * quantizer (codes and scales bit-identical). Same group order and epilogue as the GEMM
  * (acc = fma(P_g, sx_g * sw_g, acc), * s2 * second, + la . up, + bias,
  * optional GELU-tanh); only the low-rank sum rounds differently.
  *   x / smooth / s2 / proj_down_op6 / proj_up / second / bias / out /

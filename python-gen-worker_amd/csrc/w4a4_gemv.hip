@@ -275,8 +275,8 @@ __global__ __launch_bounds__(64) void svdq_la_few_rows_kernel(const uint16_t* __
   }
 }
 
-// activation records (+ 1 KB slack) and la partial slots of kernel 1, 256-byte aligned pieces
-int64_t records_bytes(int64_t M, int64_t K) { return ((K / 128) * M * GWA_FP6_REC + 1024 + 255) / 256 * 256; }
+// la's partial slots: one [M, R] fp32 block per 128-column stage, what svdq_la_few_rows_kernel's grid stores
+int64_t la_slots(int64_t K) { return K / 128; }
 
 }  // namespace
 
@@ -291,7 +291,7 @@ extern "C" int gwa_svdq_w4a4_gemv_max_m(int64_t K, int64_t rank) {
 extern "C" int64_t gwa_svdq_w4a4_linear_gemv_workspace(int64_t M, int64_t K, int64_t rank) {
   if (M <= 0 || K <= 0 || K % 128 || rank < 0) return 0;
   if (rank == 0) return 256;
-  return records_bytes(M, K) + gwa_svdq_quant_fp6_la_workspace(M, K, rank);
+  return la_slots(K) * M * rank * 4;
 }
 
 extern "C" int gwa_svdq_w4a4_linear_gemv(const void* x, int64_t ldx, const void* smooth, const float* s2,
@@ -331,11 +331,10 @@ extern "C" int gwa_svdq_w4a4_linear_gemv(const void* x, int64_t ldx, const void*
   const float* la_part = nullptr;
   int P = 0;
   if (R > 0) {
-    // la's partial slots, behind the records' place in the workspace (kernel 1's layout)
     GWA_REQUIRE(GWA_ALIGNED(proj_down_op6, 16) && M * ldx * 2 < (1ll << 31),
                 "%s: proj_down_op6 must be 16-byte aligned and x below 2 GiB (buffer addressing)", what);
-    float* part = (float*)((uint8_t*)workspace + records_bytes(M, K));
-    P = (int)(K / 128);
+    float* part = (float*)workspace;
+    P = (int)la_slots(K);
     const dim3 lgrid((unsigned)P, (unsigned)(R / 16));
     const uint16_t *lx = (const uint16_t*)x, *pd = (const uint16_t*)proj_down_op6;
 #define GWA_LA_LAUNCH(RBV) \

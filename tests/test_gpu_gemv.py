@@ -182,3 +182,27 @@ def test_low_rank_product_is_kernel_1s(m, k, rank):
                               torch.ones(n, k // 64, dtype=torch.float16, device=DEV), None, up, None,
                               torch.bfloat16, False)
     assert np.array_equal(bits16(y), bits16(torch.cat([la, la], 1)))
+
+
+@pytest.mark.parametrize("m,k,rank", [(1, 128, 16), (8, 3072, 32), (3, 8192, 128)])
+def test_workspace_holds_every_slot(m, k, rank):
+    """A workspace of exactly the stated size: the same output as a larger one's, and no byte past it written."""
+    from gen_worker_amd import _native as nat
+    from gen_worker_amd import ops
+
+    if m > ops.gemv_max_m(k, rank):
+        m = ops.gemv_max_m(k, rank)
+    g = torch.Generator().manual_seed(m + k + rank)
+    n = 64
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    pd6 = ops.svdq_prep_proj_down_fp6((torch.randn(k, rank, generator=g) * 0.05).to(torch.bfloat16).to(DEV))
+    up = torch.randn(n, rank, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8).to(DEV)
+    sw = (torch.rand(n, k // 64, generator=g) * 0.01).to(torch.float16).to(DEV)
+    need = int(nat.load().gwa_svdq_w4a4_linear_gemv_workspace(m, k, rank))
+    ws = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device=DEV)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    nat.call("gwa_svdq_w4a4_linear_gemv", nat.ptr(x), k, None, None, nat.ptr(pd6), rank, nat.ptr(w), nat.ptr(sw), None, 0,
+             nat.ptr(up), None, nat.ptr(out), 0, 0, m, n, k, nat.ptr(ws), need, nat.stream_of(x))
+    want = ops.svdq_forward_gemv(x, None, None, pd6, w, sw, None, up, None, torch.bfloat16, False)
+    assert torch.equal(out, want) and bool((ws[need:] == 0xA5).all())

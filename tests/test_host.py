@@ -206,6 +206,16 @@ def test_invalid_arguments_are_refused_before_any_launch():
     assert lib.gwa_probe_add_one(None, None, 0, None) == 0
 
 
+def test_small_m_workspace_is_the_slots_its_kernel_writes():
+    """One [M, rank] fp32 slot per 128 inputs, whatever kernel 1's split of K would be."""
+    from gen_worker_amd import _native
+
+    ws = _native.load().gwa_svdq_w4a4_linear_gemv_workspace
+    for m, k, r in ((1, 128, 16), (8, 3072, 32), (3, 8192, 128)):
+        assert ws(m, k, r) == k // 128 * m * r * 4
+    assert ws(4, 3072, 0) == 256 and ws(0, 3072, 32) == 0 and ws(1, 192, 32) == 0
+
+
 def test_record_buffer_sizes_are_checked_at_the_c_abi():
     """Every C entry point that reads fp6 records takes each record pointer's readable byte count and refuses a
     buffer shorter than the records plus GWA_FP6_RECORD_SLACK (the GEMMs' 1 KB copy runs may read that far past
