@@ -442,10 +442,9 @@ int gwa_w8a8_gemm(const int8_t* qa, const int8_t* qw, const float* sa, int64_t s
 
 /* The output tile gwa_w8a8_gemm uses for this shape (-1 for an empty shape):
  * of 256 x 256 (512 threads; K a multiple of 128 below 2^23), 128 x 128,
- * 64 (m) x 128 and 64 x 64, the one whose workgroups finish first. Returns
- * GWA_W8A8_TILE_256x256, or GWA_W8A8_TILE_128x128 for one of the smaller three;
- * the forced tile itself while one is set. No reference counterpart:
- * torch._scaled_mm picks its own kernel. */
+ * 64 (m) x 128 and 64 x 64, the one whose workgroups finish first; the forced
+ * tile while one is set. No reference counterpart: torch._scaled_mm picks its
+ * own kernel. */
 enum { GWA_W8A8_TILE_128x128 = 0, GWA_W8A8_TILE_256x256 = 1, GWA_W8A8_TILE_64x64 = 2, GWA_W8A8_TILE_64x128 = 3 };
 int gwa_w8a8_gemm_tile(int64_t M, int64_t N, int64_t K);
 

@@ -484,10 +484,7 @@ int w8a8_tile(int64_t M, int64_t N, int64_t K) {
 }  // namespace
 
 extern "C" int gwa_w8a8_gemm_tile(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0) return -1;
-  const int tile = w8a8_tile(M, N, K);
-  if (tile == GWA_W8A8_TILE_256x256 || g_w8a8_force_tile.load(std::memory_order_relaxed) >= 0) return tile;
-  return GWA_W8A8_TILE_128x128;  // the family of 128 x 128 and below
+  return M <= 0 || N <= 0 || K <= 0 ? -1 : w8a8_tile(M, N, K);
 }
 
 extern "C" int gwa_w8a8_gemm_force_tile(int tile) {

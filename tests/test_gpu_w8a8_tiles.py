@@ -134,3 +134,20 @@ def test_small_tiles_agree_and_match_oracle(force, m, n, k, pertensor, bdt, odt)
     assert all(torch.equal(o, outs[0]) for o in outs), f"tiles differ at {(m, n, k)}"
     bref = None if bdt is None else bias.float().cpu().numpy()
     check_output(outs[1], O.w8a8_linear(xb, qw, sw, bref, pertensor=pertensor), what=f"w8a8 64x64 tile {(m, n, k)}")
+
+
+@pytest.mark.parametrize("tile,m,n,k", [(0, 512, 9216, 192), (1, 4608, 3072, 128), (2, 65, 528, 256), (3, 250, 9216, 192)])
+def test_the_chosen_tile_is_the_one_the_query_names(force, tile, m, n, k):
+    from gen_worker_amd import _native
+
+    assert _native.load().gwa_w8a8_gemm_tile(m, n, k) == tile
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    qa = torch.randint(-127, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    qw = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    sa, sw = (torch.rand(t, device=DEV, generator=g) * 1e-3 + 1e-4 for t in (m, n))
+    y = torch.ops.cozy_gen_worker.w8a8_scaled_mm(qa, qw, sa, sw, None, torch.bfloat16)
+    force(tile)
+    assert torch.equal(y, torch.ops.cozy_gen_worker.w8a8_scaled_mm(qa, qw, sa, sw, None, torch.bfloat16))
+    rows = torch.arange(0, m, max(1, m // 9), device=DEV)
+    ref = ((qa[rows].double() @ qw.double().t()).float() * sa[rows, None] * sw[None, :]).double().cpu().numpy()
+    check_output(y[rows], ref, what=f"w8a8 tile {tile} {(m, n, k)}")
