@@ -621,7 +621,8 @@ __device__ __forceinline__ float w8a8_code(float v, float s) {
 // division does for every bf16 v and s = RN(amax / 127) with |v| <= amax (checked over all significands, 16
 // binades down; smaller ones round to code 0 either way); a row whose scale or values are not ordinary numbers, and a
 // static scale, take the division itself. Bound by that division and a second pass over x before (a 256-thread
-// workgroup per row: 13.0 us at 4608 x 3072; the QKV layer there 134.0 -> 127.9 us).
+// workgroup per row: 11.9 us at 4608 x 3072, this 8.2; the QKV layer there 134.0 -> 127.9 us). Which calls take it:
+// gwa_w8a8_quant.
 template <int MODE, int NC>
 __global__ __launch_bounds__(256) void w8a8_quant_int8_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                    int8_t* __restrict__ q, float* __restrict__ sa,
@@ -688,7 +689,7 @@ __global__ __launch_bounds__(256) void w8a8_quant_int8_rows_kernel(const uint16_
   if (lane == 0 && (sa_per_row || row == 0)) sa[sa_per_row ? row : 0] = s;
 }
 
-// longer rows: a 256-thread workgroup per row, read twice
+// the rest: a 256-thread workgroup per row, read twice (once for a static or per-tensor scale)
 template <int MODE>
 __global__ __launch_bounds__(256) void w8a8_quant_int8_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                               int8_t* __restrict__ q, float* __restrict__ sa,
@@ -943,15 +944,27 @@ extern "C" int gwa_w8a8_quant(const void* x, int64_t ldx, int8_t* q, float* sa, 
   const int per_row = pertensor ? 0 : 1;
   auto quantize = [&](auto mode, const float* src) {
     constexpr int MODE = decltype(mode)::value;
+    // The register kernel, or a workgroup per row that reads it twice (once where the scale is given); us below are the
+    // workgroup's and the register kernel's. A wave's row is a serial chain, so a few long rows take the workgroup
+    // (1 x 12288 4.9 and 6.1, 512 x 6152 5.1 and 5.6; 700 x 6152 5.9 and 5.9, 1000 x 6144 6.3 and 5.4, 256 x 3072 3.3
+    // and 3.3). With the scale known there is no second read to save: per tensor, the register kernel for many rows of
+    // up to 6144 (4608 x 6144 49.0 and 47.0, 4608 x 12288 67.0 and 69.6, 256 x 3072 9.1 and 9.5, 512 x 6144 13.4 and
+    // 14.0); a static scale, by which it divides, for many short rows only (16384 x 512 6.9 and 6.5, 4608 x 3072 9.7
+    // and 11.6, 4608 x 12288 27.6 and 39.5).
+    const bool in_registers = MODE == kW8Static ? K <= 512 && M >= 4096
+                              : MODE == kW8Tensor ? K <= 6144 && M >= 700
+                                                  : K <= 3072 || (K <= 12288 && M >= 700);
     const int64_t per = M < 1024 ? 1 : 4;  // rows per workgroup: few rows spread over the CUs
     const dim3 rows((unsigned)((M + per - 1) / per)), waves((unsigned)(64 * per));
 #define GWA_W8_ROWS(NC)                                                                                            \
   hipLaunchKernelGGL((w8a8_quant_int8_rows_kernel<MODE, NC>), rows, waves, 0, s, xp, ldx, q, sa, src, per_row, (int)M, \
                      (int)K)
-    if (K <= 512 * 6) GWA_W8_ROWS(6);
-    else if (K <= 512 * 12) GWA_W8_ROWS(12);
-    else if (K <= 512 * 24) GWA_W8_ROWS(24);
-    else hipLaunchKernelGGL((w8a8_quant_int8_kernel<MODE>), grid, block, 0, s, xp, ldx, q, sa, src, per_row, (int)K);
+    if (!in_registers)
+      hipLaunchKernelGGL((w8a8_quant_int8_kernel<MODE>), grid, block, 0, s, xp, ldx, q, sa, src, per_row, (int)K);
+    else if constexpr (MODE == kW8Static) GWA_W8_ROWS(1);
+    else if (K <= 512 * 6) GWA_W8_ROWS(6);
+    else if (MODE == kW8Tensor || K <= 512 * 12) GWA_W8_ROWS(12);
+    else if constexpr (MODE == kW8Row) GWA_W8_ROWS(24);
 #undef GWA_W8_ROWS
   };
   if (input_scale) {

@@ -99,29 +99,39 @@ def test_module_modes(mode, static):
     check_output(y.reshape(-1, 512), ref, what=f"module {mode} static={static}")
 
 
-
-@pytest.mark.parametrize("m,k", [(1, 64), (5, 3072), (3, 3080), (6, 6144), (2, 6152), (4, 12288), (3, 12296)])
-@pytest.mark.parametrize("pertensor,static", [(False, None), (True, None), (False, 0.037)])
+@pytest.mark.parametrize("m,k", [(1, 64), (5, 3072), (3, 3080), (6, 6144), (2, 6152), (4, 12288), (3, 12296),
+                                 (699, 3080), (701, 3072), (703, 3080), (700, 6144), (701, 6152), (702, 12288),
+                                 (701, 12296), (4095, 64), (4097, 512), (4098, 520)])
+@pytest.mark.parametrize("pertensor,static", [(False, None), (True, None), (False, 0.037), (True, 0.037)])
 def test_quantizer_at_the_ends_of_its_register_sizes(m, k, pertensor, static):
-    """Rows on either side of each register size (and the two-pass kernel past them), with a row of zeros, an infinite
-    row and a NaN: the codes and scales of the IEEE division, bit for bit."""
+    """Both sides of each register size and of the row counts that choose the kernel. Plain rows, then with an infinity, a
+    row of zeros, one whose scale is clamped to 1e-12, one of subnormal values, and a NaN (which no maximum counts):
+    the scales and the finite values' codes (0 over an infinite scale) are the IEEE division's, bit for bit."""
     g = np.random.default_rng(m * 7 + k)
     x = (g.standard_normal((m, k)) * np.exp(g.uniform(-6, 3, (m, 1)))).astype(np.float32)
     x[:, g.integers(0, k, 2)] *= 30.0
-    xb = O.f32_to_bf16_bits(x)
-    xf = O.bf16_bits_to_f32(xb)
-    rows = [xf]
+    xf = O.bf16_bits_to_f32(O.f32_to_bf16_bits(x))
+    z = xf.copy()
+    z[-1, 3] = np.inf
+    cases = [xf, z]
     if m > 2:
-        z = xf.copy()
-        z[1] = 0.0
+        z = z.copy()
+        z[0] = 0.0
+        z[1] *= 1e-10 / np.abs(z[1]).max()
+        z[3 % m] *= 2.0 ** -125 if m > 3 else 1.0
+        cases.append(z)
+        z = z.copy()
+        z[-1, 3] = 1.0
+        z[1, 5] = -np.inf
         if not pertensor:
-            z[2, 3] = np.inf
-        rows.append(z)
-    for xr in rows:
-        xd = torch.from_numpy(xr).to(torch.bfloat16).to(DEV)
+            z[2, k // 2] = np.nan
+        cases.append(z)
+    for xr in cases:
+        xr = O.bf16_bits_to_f32(O.f32_to_bf16_bits(xr))
         st = None if static is None else torch.tensor([[static]], dtype=torch.float32, device=DEV)
-        q, s = torch.ops.cozy_gen_worker.w8a8_quant(xd, pertensor, st)
-        wq, ws = O.quantize_act_int8(O.f32_to_bf16_bits(xr), pertensor, static)
+        q, s = torch.ops.cozy_gen_worker.w8a8_quant(torch.from_numpy(xr).to(torch.bfloat16).to(DEV), pertensor, st)
+        known = np.isfinite(xr)
+        with np.errstate(invalid="ignore"):
+            wq, ws = O.quantize_act_int8(O.f32_to_bf16_bits(np.where(np.isnan(xr), 0.0, xr)), pertensor, static)
         assert np.array_equal(s.cpu().numpy(), ws.reshape(s.shape))
-        fin = np.isfinite(xr).all(axis=1)   # a finite value over an infinite scale is a code 0; inf / inf is not a code
-        assert np.array_equal(q.cpu().numpy()[fin], wq[fin])
+        assert np.array_equal(q.cpu().numpy()[known], wq[known])
