@@ -31,6 +31,7 @@
 namespace {
 
 constexpr int NV_THREADS = 256;
+constexpr int kCus = 256;  // MI355X compute units
 
 // e2m1 code (sign bit 3) -> its value: magnitude m = code & 7 is 0 or 0.5 (m < 2), else
 // 2^((m >> 1) - 1) * (1 + (m & 1) / 2), built from its fp32 exponent and top mantissa bit
@@ -172,11 +173,10 @@ __device__ __forceinline__ uint32_t e2m1_pair_value(uint32_t codes, float sa) {
 // Two lanes per block (lane pair 2p, 2p + 1 holds its elements 0-7 and 8-15), so every load and store of a
 // wave covers one contiguous run; the block maximum is one exchange within the pair. A workgroup takes NV_HALVES
 // runs of 256 half-blocks, their loads issued before the partial maxima are folded. It was bound by VALU work (an IEEE
-// division and ten compares per element, a 64-bit division per half-block, one run per workgroup): 26.9 us at
-// 4608 x 3072 with codes, scales and values written; values alone 14.0 now (2 x 28 MB: 4.0 TB/s, where a plain copy
-// of the array takes 8.4 us from the cache). q and scales may both be absent (values only).
-constexpr int NV_HALVES = 4;
-
+// division and ten compares per element, a 64-bit division per half-block): 22.2 us at 4608 x 3072 with a static s2 and
+// codes, scales and values written, 11.6 now; values alone 10.6 (2 x 28 MB: 5.3 TB/s, from the cache). q and scales
+// may both be absent (values only).
+template <int NV_HALVES>
 __global__ __launch_bounds__(NV_THREADS) void nvfp4_quant_act_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                      const float* __restrict__ s2p,
                                                                      uint8_t* __restrict__ q,
@@ -348,7 +348,14 @@ static int nvfp4_quant(const char* what, const void* x, int64_t ldx, const float
     if (rc != GWA_OK) return rc;
   }
   const int64_t halves = 2 * M * (K / 16);
-  hipLaunchKernelGGL(nvfp4_quant_act_kernel, dim3((unsigned)((halves + NV_THREADS * NV_HALVES - 1) / (NV_THREADS * NV_HALVES))),
+  // Four runs a workgroup where the partial maxima's folds weigh (dynamic s2, from 25 M values on: us, one run and four,
+  // 1024 x 1024 6.0 and 7.8, 4608 x 3072 20.2 and 21.5, 8192 x 3072 33.7 and 33.3, 16384 x 12288 289 and 246), and for
+  // codes alone past the cache (100 M: 8192 x 15360 79.6 and 70.7); otherwise one (1024 x 1024 2.9 and 4.6, 4608 x 3072
+  // 11.6 and 13.2, 16384 x 12288 150 and 161).
+  const int64_t runs_per_cu = halves / ((int64_t)NV_THREADS * kCus);
+  const bool four = parts ? runs_per_cu >= 48 : !xdq && runs_per_cu >= 192;
+  const int64_t run = NV_THREADS * (four ? 4 : 1);
+  hipLaunchKernelGGL(four ? nvfp4_quant_act_kernel<4> : nvfp4_quant_act_kernel<1>, dim3((unsigned)((halves + run - 1) / run)),
                      dim3(NV_THREADS), 0, st, (const uint16_t*)x, ldx, s2, q, scales,
                      scale_layout == GWA_NVFP4_SCALES_BLOCKED ? 1 : 0, (uint16_t*)xdq, M, (int)(K / 16), parts,
                      nparts, s2_out);

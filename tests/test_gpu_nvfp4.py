@@ -231,6 +231,31 @@ def test_values_alone_equal_the_quantizers(m, k):
         assert torch.equal(v, dyn) and torch.equal(s, s2d)
 
 
+@pytest.mark.parametrize("m,k", [(8192, 3072), (8191, 3088), (1541, 16400)])
+def test_workgroups_of_four_runs_equal_those_of_one(m, k):
+    """Either side of 25 M values, where the quantizer with a dynamic second scale goes over to four runs a workgroup:
+    the static quantizer's bits at that scale (one run, compared with the oracle above), flat and blocked."""
+    cg = torch.ops.cozy_gen_worker
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x = torch.randn(m, k, generator=g, device=DEV).to(torch.bfloat16)
+    for blocked in (False, True):
+        q, sc, xdq, s2 = cg.nvfp4_quant_act_dyn(x, blocked, True)
+        q0, sc0, xdq0 = cg.nvfp4_quant_act(x, s2, blocked, True)
+        assert torch.equal(q, q0) and torch.equal(sc, sc0) and torch.equal(xdq, xdq0)
+    assert torch.equal(cg.nvfp4_act_values(x, None)[0], xdq0)
+
+
+@pytest.mark.parametrize("m,k", [(8193, 12288), (6131, 16400)])
+def test_codes_alone_equal_the_codes_beside_values(m, k):
+    """Either side of 100 M values, where codes alone go over to four runs a workgroup."""
+    cg = torch.ops.cozy_gen_worker
+    x = torch.randn(m, k, generator=torch.Generator(device=DEV).manual_seed(m), device=DEV).to(torch.bfloat16)
+    s2 = torch.tensor(0.0021, device=DEV)
+    q, sc, _ = cg.nvfp4_quant_act(x, s2, True, False)
+    q0, sc0, _ = cg.nvfp4_quant_act(x, s2, True, True)
+    assert torch.equal(q, q0) and torch.equal(sc, sc0)
+
+
 @pytest.mark.parametrize("m,n", [(1, 8), (3, 136), (65, 2056), (130, 4096)])
 def test_scale_bias_tile_ends(m, n):
     g = np.random.default_rng(m + n)
