@@ -265,16 +265,17 @@ __global__ __launch_bounds__(NV_THREADS) void nvfp4_dequant_kernel(const uint8_t
 // `y * (s2 * weight_scale_2).to(y.dtype)` then `+ bias` (models/w4a4.py:349-351), each rounded to bf16 as
 // torch's bf16 ops round. A workgroup is tx (columns of 8) x ty threads (a power of two each) and takes SB_ROWS rows
 // of every thread's column: the bias is loaded once for them, their loads are in flight together, and no column is
-// found by a 64-bit remainder (12.1 us at 4608 x 3072 with one column of one row per thread, 10.5 so).
-constexpr int SB_ROWS = 4;
-
+// found by a 64-bit remainder (9.2 us at 4608 x 3072 with one column of one row per thread, 7.3 so). Workgroups go
+// along the rows first: past the cache, memory likes whole rows (16384 x 12288 150 us going down the columns, 134 so).
+template <int SB_ROWS>
 __global__ __launch_bounds__(NV_THREADS) void nvfp4_scale_bias_kernel(uint16_t* __restrict__ y,
                                                                       const float* __restrict__ s2,
                                                                       const float* __restrict__ ws2,
                                                                       const uint16_t* __restrict__ bias, int64_t M,
-                                                                      int N) {
-  const int n = 8 * (int)(blockIdx.y * blockDim.x + threadIdx.x);
-  const int64_t r0 = ((int64_t)blockIdx.x * SB_ROWS) * blockDim.y + threadIdx.y;
+                                                                      int N, unsigned ncols) {
+  const unsigned rb = blockIdx.x / ncols, cb = blockIdx.x - rb * ncols;
+  const int n = 8 * (int)(cb * blockDim.x + threadIdx.x);
+  const int64_t r0 = ((int64_t)rb * SB_ROWS) * blockDim.y + threadIdx.y;
   if (n >= N || r0 >= M) return;
   v4i w[SB_ROWS];
 #pragma unroll
@@ -309,12 +310,19 @@ extern "C" int gwa_nvfp4_scale_bias(void* y, const float* s2, const float* ws2, 
               "%s: y and bias must be 16-byte aligned", what);
   int tx = 16;
   while (tx < NV_THREADS && tx < N / 8) tx *= 2;
+  if (tx == NV_THREADS && (N / 8 - 1) % tx < tx / 2) tx /= 2;  // fewer idle columns (3072: 384 of 384 instead of 512)
   const int ty = NV_THREADS / tx;
-  const int64_t gx = (M + SB_ROWS * ty - 1) / (SB_ROWS * ty), gy = (N / 8 + tx - 1) / tx;
-  GWA_REQUIRE(gx < (1ll << 31) && gy < 65536 && N < (1ll << 31), "%s: [%lld, %lld] is too large", what, (long long)M,
+  const int64_t nc = (N / 8 + tx - 1) / tx;
+  // four rows a thread from three such workgroups per CU on (6.3 M values; us, one row and four: 64 x 3072 2.3 and 2.8,
+  // 1024 x 3072 3.5 and 3.8, 2048 x 3072 5.1 and 5.1, 4608 x 3072 8.3 and 7.3)
+  const bool four = (M + 4 * ty - 1) / (4 * ty) * nc >= 3 * kCus;
+  const int rows = (four ? 4 : 1) * ty;
+  const int64_t blocks = (M + rows - 1) / rows * nc;
+  GWA_REQUIRE(blocks < (1ll << 31) && N < (1ll << 31), "%s: [%lld, %lld] is too large", what, (long long)M,
               (long long)N);
-  hipLaunchKernelGGL(nvfp4_scale_bias_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(tx, ty), 0, (hipStream_t)stream,
-                     (uint16_t*)y, s2, ws2, (const uint16_t*)bias, M, (int)N);
+  hipLaunchKernelGGL(four ? nvfp4_scale_bias_kernel<4> : nvfp4_scale_bias_kernel<1>, dim3((unsigned)blocks),
+                     dim3(tx, ty), 0, (hipStream_t)stream, (uint16_t*)y, s2, ws2, (const uint16_t*)bias, M, (int)N,
+                     (unsigned)nc);
   return gwa_check_launch(what);
 }
 

@@ -256,7 +256,8 @@ def test_codes_alone_equal_the_codes_beside_values(m, k):
     assert torch.equal(q, q0) and torch.equal(sc, sc0)
 
 
-@pytest.mark.parametrize("m,n", [(1, 8), (3, 136), (65, 2056), (130, 4096)])
+# the last three: either side of 768 workgroups of four rows a thread, and one column block that is not full
+@pytest.mark.parametrize("m,n", [(1, 8), (3, 136), (65, 2056), (130, 4096), (2047, 3072), (2045, 3080), (12301, 520)])
 def test_scale_bias_tile_ends(m, n):
     g = np.random.default_rng(m + n)
     y = N.bf16_round((g.standard_normal((m, n)) * 3).astype(np.float32))
