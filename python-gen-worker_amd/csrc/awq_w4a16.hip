@@ -28,7 +28,7 @@
 //    activation row (fp32 accumulation), the activations read as 16 bytes
 //    per lane from LDS, swizzled so the 16 lanes of a team hit distinct banks;
 //  * the activations are requested before the weights, so that staging them
-//    waits for them alone, and every span of a row of up to 4096 inputs is
+//    waits for them alone, and every span of a row of up to 6144 inputs is
 //    requested at once (longer rows: batches of 4 spans, two in flight); the
 //    team's 16 partial sums are reduced by lane exchanges, and lane 0 adds the
 //    bias and stores the bf16 result.
@@ -42,7 +42,7 @@ namespace {
 constexpr int AWQ_THREADS = 256, AWQ_TEAMS = AWQ_THREADS / 16;  // 16 output rows per workgroup
 constexpr int AWQ_SPAN = 512;                                    // codes of a row per team step (16 lanes x 32)
 constexpr int AWQ_BATCH = 4;                                     // spans per load batch of a long row
-constexpr int AWQ_ALL = 8;                                       // rows of up to this many spans load at once
+constexpr int AWQ_ALL = 12;                                      // rows of up to this many spans load at once
 constexpr int AWQ_MFMA_SPAN = 128;                                // codes of a row per wave step of the MFMA kernel
 constexpr int AWQ_LDS_MAX = 64 * 1024;                           // activation rows staged in LDS
 
@@ -86,7 +86,7 @@ __device__ __forceinline__ void barrier_staged() {
 // the other. us, before -> now: 3072 -> 18432, 1 row 11.8 -> 9.7, 2 13.7 -> 11.8, 4 17.8 -> 15.8; 12288 -> 3072, 1 row
 // 14.1 -> 10.4; 15360 -> 18432, 4 rows 117 -> 94. What is left at one row: 3.9 us of launch and staging, 3.5 of loads
 // and 4.5 of arithmetic, now partly over one another.
-template <int MT, int B, bool PIPED>
+template <int MT, int B, bool PIPED, int XU>
 __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint8_t* __restrict__ weight,
     const uint16_t* __restrict__ wscales, const uint16_t* __restrict__ wzeros, const uint16_t* __restrict__ bias,
@@ -109,9 +109,7 @@ __global__ __launch_bounds__(AWQ_THREADS) void awq_w4a16_gemv_kernel(
   const uint32_t grow = (uint32_t)((int64_t)n * ng + (t >> 1)) * 2u;
 
   // 1. the MT activation rows (rows past M: zeros): the first XU units of each thread into registers, ahead of the
-  //    weights (that is all of them up to K = 16384; long rows with 2 MT units ahead instead:
-  //    12288 -> 3072 11.4 us for 10.4, 15360 -> 512 in chunks of two rows 18.8 for 17.6)
-  constexpr int XU = PIPED ? (MT == 1 ? 8 : 16) : (MT * B + 3) / 4;
+  //    weights (launch_gemv: all of them, as far as registers go)
   auto x_load = [&](int u) __attribute__((always_inline)) {
     const int r = u / ku, c = u - r * ku;
     return buf_load16(xbuf, u < MT * ku && m0 + r < M ? (uint32_t)(((int64_t)(m0 + r) * ldx + 8 * c) * 2) : kOOB);
@@ -266,8 +264,11 @@ __global__ __launch_bounds__(256) void awq_w4a16_dequant_kernel(const uint32_t* 
   *(v4i*)(out + 8 * i) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
-// rows of up to AWQ_ALL spans load whole (three batch sizes, so that a short row does not issue loads for spans it does
-// not have)
+// Rows of up to AWQ_ALL spans load whole (several batch sizes, so that a row does not issue loads for many spans it does
+// not have: two rows 4224 -> 3072 pipelined 8.3 us, 12 spans at once 7.5, 10 7.4; 6144 -> 3072 9.6 and 8.9; 16 at once
+// for 8192 11.4, pipelined 10.8). Units of activations ahead of the weights: all of a thread's, which is a whole row
+// of up to 16384 in 8 (with 2 ahead 12288 -> 3072 took 11.4 us for 10.4; chunks of two rows with 4, 15360 -> 512 18.8
+// for 17.6, with 8 18.1), but no more than there are (two rows 8192 -> 3072 with 16 11.1, with their 8 10.8).
 template <int MT>
 int launch_gemv(const void* x, int64_t ldx, const void* weight, const void* ws, const void* wz, const void* bias,
                 void* out, int64_t M, int64_t N, int64_t K, hipStream_t st) {
@@ -279,11 +280,18 @@ int launch_gemv(const void* x, int64_t ldx, const void* weight, const void* ws, 
                        (const uint16_t*)ws, (const uint16_t*)wz, (const uint16_t*)bias, (uint16_t*)out, (int)M, (int)N,
                        (int)K);
   };
-  if (spans > AWQ_ALL) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH, true>);
-  else if (spans > AWQ_BATCH + 2) go(awq_w4a16_gemv_kernel<MT, AWQ_ALL, false>);
-  else if (spans > AWQ_BATCH) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH + 2, false>);
-  else if (spans > AWQ_BATCH - 2) go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH, false>);
-  else go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH - 2, false>);
+#define GWA_AWQ_WHOLE(B) go(awq_w4a16_gemv_kernel<MT, B, false, (MT * B + 3) / 4>)
+  if (spans > AWQ_ALL) {
+    if constexpr (MT == 1) go(awq_w4a16_gemv_kernel<1, AWQ_BATCH, true, 8>);
+    else if (MT == 2 && K <= 8192) go(awq_w4a16_gemv_kernel<2, AWQ_BATCH, true, 8>);
+    else go(awq_w4a16_gemv_kernel<MT, AWQ_BATCH, true, 16>);
+  } else if (spans > 10) GWA_AWQ_WHOLE(AWQ_ALL);
+  else if (spans > 8) GWA_AWQ_WHOLE(10);
+  else if (spans > 6) GWA_AWQ_WHOLE(8);
+  else if (spans > 4) GWA_AWQ_WHOLE(6);
+  else if (spans > 2) GWA_AWQ_WHOLE(4);
+  else GWA_AWQ_WHOLE(2);
+#undef GWA_AWQ_WHOLE
   return gwa_check_launch("awq_w4a16_mm");
 }
 

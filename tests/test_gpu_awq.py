@@ -53,10 +53,10 @@ def test_mm_matches_oracle(m, n, k, bias):
     check_output(y, ref, what=f"awq m={m} n={n} k={k} ({'gemv' if m <= AWQ_GEMV_MAX_M else 'dequant + gemm'})")
 
 
-@pytest.mark.parametrize("k", [1024, 1152, 2048, 2176, 3200, 4096, 4224, 8320, 15360])
+@pytest.mark.parametrize("k", [1024, 1152, 2048, 2176, 3200, 4096, 4224, 5120, 5248, 6144, 6272, 8192, 8320, 15360])
 @pytest.mark.parametrize("m", [1, 2, 4])
 def test_mm_load_batches(m, k):
-    """Rows on both sides of each load batch (2, 4, 6 and 8 spans of 512 held at once, longer rows pipelined) and of
+    """Rows on both sides of each load batch (2 to 12 spans of 512 held at once, longer rows pipelined) and of
     the activations requested ahead of the weights; N = 48 leaves no full multiple of 64 rows."""
     codes, s, z, b, t = _layer(48, k, seed=m + k)
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(m + k)).to(torch.bfloat16)
