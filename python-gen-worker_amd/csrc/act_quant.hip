@@ -7,7 +7,8 @@
 
 // ---------------------------------------------------------------------------
 // Kernel 1: smoothing divide -> group-64 absmax -> fp16 scale -> int4 codes;
-// plus la = x @ proj_down on the RAW activations via bf16 MFMA 16x16x32.
+// plus la = x @ proj_down on the RAW activations via bf16 MFMA 16x16x32
+// (without a low-rank product: svdq_quant_int4_rows_kernel).
 //
 // Work split: a 512-thread workgroup owns 16 rows and walks K in rounds of
 // 256 columns (4 groups). Each round's 16 x 256 bf16 tile is loaded with
@@ -54,7 +55,6 @@ __global__ __launch_bounds__(512) void svdq_quant_int4_kernel(
     const float* __restrict__ s2p, const uint16_t* __restrict__ pdo, uint8_t* __restrict__ q,
     uint16_t* __restrict__ sc, uint16_t* __restrict__ la, int M, int K) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int RBX = RB > 0 ? RB : 1;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int row0 = blockIdx.x * 16;
   const int G = K >> 6;
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(512) void svdq_quant_int4_kernel(
   struct Slot {
     v4i xv;
     uint32_t sv;
-    v4i lo[RBX];
+    v4i lo[RB];
   };
   auto load_tile = [&](Slot& s, int r) {
     const int kb = r * KT;
@@ -120,13 +120,13 @@ __global__ __launch_bounds__(512) void svdq_quant_int4_kernel(
 #pragma unroll
   for (int j = 0; j < PF; ++j) {
     load_tile(slot[j], j);
-    if (RB > 0) load_lowrank(slot[j], j);
+    load_lowrank(slot[j], j);
   }
   __syncthreads();
 
-  v4f acc[RBX];
+  v4f acc[RB];
 #pragma unroll
-  for (int rb = 0; rb < RBX; ++rb) acc[rb] = (v4f){0.f, 0.f, 0.f, 0.f};
+  for (int rb = 0; rb < RB; ++rb) acc[rb] = (v4f){0.f, 0.f, 0.f, 0.f};
 
   for (int rr = 0; rr < rounds; rr += PF) {
 #pragma unroll
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(512) void svdq_quant_int4_kernel(
       }
 
       // ---- la += x[:, slice] @ proj_down[slice, :] for this wave's 32-column slice
-      if (RB > 0) {
+      {
         const v4i a = *(const v4i*)(base + (lane & 15) * XT_STR + wave * 64 + (lane >> 4) * 16);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -178,25 +178,23 @@ __global__ __launch_bounds__(512) void svdq_quant_int4_kernel(
     }
   }
 
-  if (RB > 0) {
-    // sum the 8 waves' partial la blocks through LDS; wave 0 writes bf16
-    __syncthreads();
-    float* lap = (float*)lds;
+  // sum the 8 waves' partial la blocks through LDS; wave 0 writes bf16
+  __syncthreads();
+  float* lap = (float*)lds;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) *(v4f*)(lap + ((wave * RB + rb) * 64 + lane) * 4) = acc[rb];
-    __syncthreads();
-    if (wave == 0) {
-      const int R = RB * 16;
+  for (int rb = 0; rb < RB; ++rb) *(v4f*)(lap + ((wave * RB + rb) * 64 + lane) * 4) = acc[rb];
+  __syncthreads();
+  if (wave == 0) {
+    const int R = RB * 16;
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        v4f s = acc[rb];
+    for (int rb = 0; rb < RB; ++rb) {
+      v4f s = acc[rb];
 #pragma unroll
-        for (int w2 = 1; w2 < 8; ++w2) s += *(const v4f*)(lap + ((w2 * RB + rb) * 64 + lane) * 4);
+      for (int w2 = 1; w2 < 8; ++w2) s += *(const v4f*)(lap + ((w2 * RB + rb) * 64 + lane) * 4);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int r = row0 + 4 * (lane >> 4) + t;
-          if (r < M) la[(int64_t)r * R + rb * 16 + (lane & 15)] = f32_to_bf16(s[t]);
-        }
+      for (int t = 0; t < 4; ++t) {
+        const int r = row0 + 4 * (lane >> 4) + t;
+        if (r < M) la[(int64_t)r * R + rb * 16 + (lane & 15)] = f32_to_bf16(s[t]);
       }
     }
   }
