@@ -457,7 +457,10 @@ int64_t w8a8_tiles(int tile, int64_t M, int64_t N) {
 }
 
 // The tile that finishes first: the most workgroups a CU gets, in batches of as many as it holds, at the batch
-// times above (they scale with K alike, so their order holds at any K). Measured at the picks against 128 x 128
+// times above. They are those of K = 3072, and a launch's and an epilogue's share does not grow with K, but their
+// order held: of 572 shapes (M 1 to 16384, N 512 to 18432, K 64 to 15360) the pick took more than 5 % over the
+// fastest tile at 55 and 12 % at most (one row 18432 x 15360: 57.4 us, 64 x 64 51.1; 118.6 the kernel before), spread
+// over all K. Measured at the picks against 128 x 128
 // for everything below 256 x 256's grids, register-staged (the form before): 256 x 3072 x 3072 64 x 64 8.5 us
 // (22.3), 256 x 9216 64 x 128 16.1 (24.4), 1024 x 3072 64 x 128 15.5 (24.5), 512 x 9216 128 x 128 22.6 (29.1),
 // 2048 x 3072 128 x 128 23.7 (31.6), K = 12288 at 256 x 3072 64 x 64 26.7 (83.6). 256 x 256's stages need
