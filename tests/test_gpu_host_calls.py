@@ -135,10 +135,30 @@ def test_awq_layer_equals_the_operator(bias):
         mod(x3.float())
 
 
+def _layer(kind, n=272, k=448):
+    from gen_worker_amd import synthetic
+    from gen_worker_amd.svdq import build_svdq_w4a4_linear
+    from gen_worker_amd.w8a8 import build_int8_linear
+
+    if kind == "awq":
+        return _awq(n, 384), 384
+    if kind == "w8a8":
+        w8 = synthetic.w8a8_layer(n, k)
+        return build_int8_linear(qweight=w8.qweight, weight_scale=w8.weight_scale, bias=w8.bias, device=DEV), k
+    k = 512 if kind == "w4a4_gemv" else k
+    _, layer = _operands(4, n, k, 32)
+    return build_svdq_w4a4_linear(qweight=layer.qweight, wscales=layer.wscales, smooth=layer.smooth,
+                                  proj_down=layer.proj_down, proj_up=layer.proj_up, bias=layer.bias, device=DEV), k
+
+
+KINDS = ["w4a4", "w4a4_gemv", "w8a8", "awq"]
+
+
 @pytest.mark.parametrize("kind", ["w4a4", "w8a8"])
 def test_layers_native_call_follows_the_module(kind):
-    """After the first forward the native call runs; an operand of another shape or device under the same attribute,
-    a LoRA addend, an in-place weight update and a mode all leave it for the general path."""
+    """After the first forward the native call runs; autograd, a mode, another activation, an in-place weight update, a
+    LoRA addend and another object or storage under an operand's attribute all leave it for the general path, also one
+    of another shape or device, which that path refuses."""
     from gen_worker_amd import synthetic
     from gen_worker_amd.svdq import build_svdq_w4a4_linear
     from gen_worker_amd.w8a8 import build_int8_linear
@@ -181,10 +201,42 @@ def test_layers_native_call_follows_the_module(kind):
         assert _same(mod(x), ref + mod._lora_addend(x))
         mod.lora_a = mod.lora_b = None
         assert _same(mod(x), ref)
-    bias = mod.bias
+    bias, data = mod.bias, mod.bias.data
     mod.bias = None
     assert native.run(x, mod.__dict__) is None
     mod.bias = bias
+    mod(x)
+    native = mod._bound.native
+    assert native.run(x, mod.__dict__) is not None
+    for other in (torch.cat([data, data]), data.cpu()):
+        bias.data = other   # the same Parameter
+        assert native.run(x, mod.__dict__) is None
+        with pytest.raises(Exception, match="bias|device|cpu"):
+            mod(x)
+    bias.data = data
+    assert native.run(x, mod.__dict__) is not None
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_native_calls_run_on_the_current_stream(kind):
+    """Queued behind what the caller's stream still has to write, not on the default stream."""
+    mod, k = _layer(kind)
+    g = torch.Generator(device=DEV).manual_seed(13)
+    a, b = (torch.randn(4, k, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    mod(a)
+    want = mod(b)
+    big = torch.randn(4096, 4096, generator=g, device=DEV)
+    x = a.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(4):
+            big = torch.sin(big @ big)   # some milliseconds before x is written
+        x.copy_(b)
+        got = mod(x)
+        got2 = got.clone()
+    side.synchronize()
+    assert _same(got, want) and _same(got2, want)
 
 
 @pytest.mark.parametrize("m,k", [(1, 64), (3, 448), (4, 512), (5, 576), (130, 1600)])
@@ -213,25 +265,6 @@ def test_quantizer_without_a_low_rank_product_equals_the_oracle(m, k, smooth):
         nat.call("gwa_svdq_quant_int4", a.data_ptr(), a.stride(0), nat.ptr(smd), one.data_ptr(), None, 0, nat.QFMT_INT4,
                  q.data_ptr(), s.data_ptr(), None, m, k, nat.stream_of(a))
         assert np.array_equal(q.cpu().numpy(), want_q) and np.array_equal(bits(s.cpu()), want_s.view(np.uint16))
-
-
-def _layer(kind, n=272, k=448):
-    from gen_worker_amd import synthetic
-    from gen_worker_amd.svdq import build_svdq_w4a4_linear
-    from gen_worker_amd.w8a8 import build_int8_linear
-
-    if kind == "awq":
-        return _awq(n, 384), 384
-    if kind == "w8a8":
-        w8 = synthetic.w8a8_layer(n, k)
-        return build_int8_linear(qweight=w8.qweight, weight_scale=w8.weight_scale, bias=w8.bias, device=DEV), k
-    k = 512 if kind == "w4a4_gemv" else k
-    _, layer = _operands(4, n, k, 32)
-    return build_svdq_w4a4_linear(qweight=layer.qweight, wscales=layer.wscales, smooth=layer.smooth,
-                                  proj_down=layer.proj_down, proj_up=layer.proj_up, bias=layer.bias, device=DEV), k
-
-
-KINDS = ["w4a4", "w4a4_gemv", "w8a8", "awq"]
 
 
 @pytest.mark.parametrize("kind", KINDS)
