@@ -673,9 +673,11 @@ def eager_call_ok(x2: Tensor) -> bool:
     """Whether a module forward may call a bound linear (``BoundLinearFp6``) instead of the registered op: a plain
     CUDA tensor, eager mode (not under torch.compile or torch.jit tracing, no Python dispatch or torch-function
     mode active, which the op would pass through), no autograd graph to record (the op has no autograd
-    formula) and no lazy negation (which the dispatcher carries out before the op reads the storage)."""
+    formula), and neither a functorch wrapper (no storage) nor a lazy negation, which the dispatcher resolves before
+    the op reads the storage."""
     return (type(x2) is Tensor and x2.is_cuda and not torch.compiler.is_compiling() and not torch._C._is_tracing()
             and not (x2.requires_grad and torch.is_grad_enabled()) and not x2.is_neg()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x2)
             and not torch._C._is_torch_function_mode_enabled()
             and torch._C._len_torch_dispatch_stack() == 0)
 

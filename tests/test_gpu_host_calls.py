@@ -360,3 +360,13 @@ def test_layers_without_the_native_host_calls(monkeypatch):
             mod._bound = None
             assert _same(mod(x), want) and _same(mod(x), want), kind
             assert mod._bound is None or mod._bound.native is None
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_layers_under_vmap(kind):
+    """A batched activation has no storage to hand to the library: the operator's own batching runs."""
+    mod, k = _layer(kind)
+    x = torch.randn(3, 4, k, generator=torch.Generator(device=DEV).manual_seed(17), device=DEV).to(torch.bfloat16)
+    mod(x[0])
+    want = torch.stack([mod(t) for t in x])
+    assert _same(torch.vmap(mod)(x), want)
